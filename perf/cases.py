@@ -334,7 +334,12 @@ def work(case):
 
 def tolerance(case):
     # 32-bit sums: four times what the products and row kernels are off 64 bits,
-    # and for `lm` what a whole run of optimizer steps is
+    # and for `lm` what a whole run of optimizer steps is.  AdamW's first steps
+    # move a weight by lr * sign(gradient), so the few weights whose gradient is
+    # near zero move the other way after any change of rounding: a few steps of
+    # 1e-4 on weights of 0.02
+    if case["kind"] == "lm" and case["opt"] == "adamw":
+        return {"rel": 5e-6, "max": 0.05}
     return {"linear": {"rel": 4e-6}, "decode": {"rel": 2e-6}, "head": {"rel": 4e-6}, "attention": {"rel": 4e-6},
             "rows": {"rel": 4e-6}, "embed": {"rel": 4e-6}, "lm": {"rel": 5e-6}, "host": {"rel": 2e-6}}[case["kind"]]
 
