@@ -159,7 +159,8 @@ LHIP_API int lhip_is_recording(void);
 LHIP_API int lhip_ktimer_start(int capacity);
 LHIP_API int lhip_ktimer_stop(float* ms, int capacity, int* count);
 
-/* ---- GEMM family (fp32 on v_mfma_f32_32x32x2f32) ---------------------------
+/* ---- GEMM family (fp32: on the fp32 matrix cores, or on the bf16 ones with
+ * each operand held exactly in three bf16 terms) -----------------------------
  * C(m x n) = alpha * op(A)(m x k) * op(B)(k x n) + beta * C, row-major.
  *   transa == 0: A is m x k, lda >= k;   transa != 0: A is stored k x m, lda >= m
  *   transb == 0: B is k x n, ldb >= n;   transb != 0: B is stored n x k, ldb >= k

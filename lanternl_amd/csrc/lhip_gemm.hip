@@ -7,31 +7,24 @@
 // (ai/gpu/luaTL_train.lua:154-182), and the host-table products of
 // ai/core/matrix.lua (multiply :541, matmul_nt :597, matmul_tn :627).
 //
-// Design (gfx950):
-//   * a workgroup of 4 wave64s computes a BM x BN tile; each wave owns a
-//     (BM/2) x (BN/2) sub-tile made of 32x32 MFMA blocks whose accumulators
-//     stay in registers for the whole K loop;
-//   * both operands are staged in LDS K-major (As[k][m], Bs[k][n]) so that one
-//     MFMA operand fetch is a single ds_read_b32 in which lanes 0-31 read 32
-//     consecutive floats of row k and lanes 32-63 those of row k+1 -- exactly
-//     the A (32x2) / B (2x32) fragment layout of v_mfma_f32_32x32x2f32;
-//   * global->LDS loads are 128-bit and coalesced along the contiguous
-//     dimension of each operand; a transposed operand is transposed on the
-//     LDS write (4 ds_write_b32 per float4), never by a separate pass; the
-//     transposing stores use an odd LDS row stride so that the 32 lanes of a
-//     half-wave hit 32 distinct banks;
-//   * two LDS buffers: the next K tile is fetched into registers while the
-//     current one feeds the MFMAs, one barrier per K tile;
-//   * workgroup ids are remapped so that consecutive tiles of a row band land
-//     on the same XCD (blocks are dispatched round-robin over the 8 XCDs, each
-//     with its own L2), then grouped GROUP_M bands at a time for L2 reuse.
-// Edge tiles (any M, N, K) use bounds-checked scalar loads with zero fill and
-// checked stores; unaligned operands (ld % 4 != 0 or a base not 16-byte
-// aligned) always take the scalar path.
+// This file holds the dispatch (sgemm_run), the fp32-core kernels of the small
+// and skinny products, the grouped weight gradients and the ordered split-K
+// reduce; everything larger runs on the three-term bf16 kernel of
+// lhip_gemm_x3.hip.  By rule (each with its measurements at the rule):
+//   * up to 16 rows of C (32 on a large aligned B), B stored K x N: one
+//     streaming pass over B (skinny_best);
+//   * fewer 32x32 tiles than CUs: 16x16 tiles, K split over the waves of a
+//     workgroup (tiny_best);
+//   * at most one 64x64 tile per CU over a short aligned K: 64x64 tiles on two
+//     wave sets (ks_best);
+//   * otherwise lhip_gemm_x3.hip's tile and split (x3_plan).
+// The workgroup ids of a product are remapped so that consecutive tiles of a row
+// band land on the same XCD (blocks are dispatched round-robin over the 8 XCDs,
+// each with its own L2), then grouped kGroupM bands at a time for L2 reuse.
 #include <algorithm>
 #include <type_traits>
 
-#include "lhip_internal.h"
+#include "lhip_gemm.h"
 #include "lhip_reduce.h"
 
 namespace lhip {
@@ -52,28 +45,6 @@ struct TileRegs {
     static constexpr int PASSES = ROWS / RPP;
     static_assert(COLS % 4 == 0 && kThreads % CQ == 0 && ROWS % RPP == 0, "tile/thread mismatch");
     float4 v[PASSES];
-
-    __device__ __forceinline__ void load(const float* __restrict__ g, int ld, int r0, int c0,
-                                         int rmax, int cmax, bool vec, int tid)
-    {
-        const int cq = tid % CQ;
-        const int rr = tid / CQ;
-        const int gc = c0 + 4 * cq;
-#pragma unroll
-        for (int p = 0; p < PASSES; ++p) {
-            const int gr = r0 + rr + p * RPP;
-            const float* src = g + static_cast<long long>(gr) * ld + gc;
-            if (vec && gr < rmax && gc + 3 < cmax) {
-                v[p] = *reinterpret_cast<const float4*>(src);
-            } else {
-                const bool rok = gr < rmax;
-                v[p].x = (rok && gc + 0 < cmax) ? src[0] : 0.f;
-                v[p].y = (rok && gc + 1 < cmax) ? src[1] : 0.f;
-                v[p].z = (rok && gc + 2 < cmax) ? src[2] : 0.f;
-                v[p].w = (rok && gc + 3 < cmax) ? src[3] : 0.f;
-            }
-        }
-    }
 
     // Every element in bounds and the stored rows 16-byte aligned: one
     // unconditional float4 load per pass (no branch for a wait to be
@@ -120,39 +91,6 @@ struct TileRegs {
             lds[(4 * cq + 3) * LD + r] = v[p].w;
         }
     }
-};
-
-// Map the linear workgroup id to a (tile_m, tile_n) pair: XCD-contiguous
-// chunks, then GROUP_M-row-band grouped raster inside the chunk order.
-__device__ __forceinline__ void tile_coords(int pid, int nwg, int tiles_m, int tiles_n, int& tm, int& tn)
-{
-    constexpr int kXcds = 8;
-    constexpr int kGroupM = 8;
-    if ((nwg % kXcds) == 0) pid = (pid % kXcds) * (nwg / kXcds) + pid / kXcds;
-    const int per_group = kGroupM * tiles_n;
-    const int group = pid / per_group;
-    const int first_m = group * kGroupM;
-    const int gsz = min(tiles_m - first_m, kGroupM);
-    const int in_group = pid - group * per_group;
-    tm = first_m + in_group % gsz;
-    tn = in_group / gsz;
-}
-
-// Kernel arguments (one struct: the launch passes it by value).
-struct GemmArgs {
-    int M, N, K;
-    float alpha, beta;
-    const float* A; int lda; long long sA, sA2;
-    const float* B; int ldb; long long sB, sB2;
-    float* C; int ldc; long long sC, sC2;
-    const float* R; int ldr;          // the beta term reads R (R == C unless a residual is given)
-    int tiles_m, tiles_n, vecA, vecB, inner;
-    int splits, kchunk;               // split-K: blockIdx.z = slice, K range [z*kchunk, (z+1)*kchunk)
-    float* ws;                        // split-K partials [split][batch][M][N]
-    int Kb;                           // batch-reduce: K = kblocks * Kb, block j reads A + j*sAk, B + j*sBk
-    long long sAk, sBk;
-    int skip_reduce;                  // split-K slices stay in ws for the caller to sum
-    size_t ws_floats_avail;           // floats available at ws (skinny path's split plan)
 };
 
 // C = alpha * sum_s ws[s] + beta * R, the slices summed in order (deterministic).
@@ -216,155 +154,22 @@ splitk_reduce4(const GemmArgs g)
     }
 }
 
-template <int BM, int BN, int BK, bool TA, bool TB>
-__global__ void __launch_bounds__(kThreads)
-sgemm_mfma_kernel(const GemmArgs g)
-{
-    constexpr int WM = BM / 2, WN = BN / 2;        // 2x2 waves
-    constexpr int FM = WM / 32, FN = WN / 32;      // 32x32 MFMA blocks per wave
-    static_assert(FM >= 1 && FN >= 1 && BK % 2 == 0, "bad tile");
-    // K-major LDS tiles.  Transposing stores want an odd row stride; direct
-    // float4 stores want a multiple of 4.
-    constexpr int LDA = TA ? BM + 4 : BM + 1;
-    constexpr int LDB = TB ? BN + 1 : BN + 4;
-    __shared__ float As[2][BK * LDA];
-    __shared__ float Bs[2][BK * LDB];
+// 64x64 tiles on two wave sets per workgroup (512 threads): set s takes the
+// 32-deep K chunks s, s + 2, ... with its own double-buffered LDS, so each SIMD
+// holds two waves and each set's chain of dependent chunk loads is half as
+// long; the sets' partial tiles meet in LDS (fixed order).  Two register sets
+// per wave set: chunk kt + 4 is in flight while chunk kt runs and chunk kt + 2
+// goes to LDS.  Every load is unconditional (past its last chunk a set reloads
+// that chunk and never stores it), so the wait before an LDS store counts only
+// the loads of the chunk being stored.
+constexpr int kKsTile = 64, kKsK = 32;
 
-    const int M = g.M, N = g.N;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int lr = lane & 31;   // row (A) / column (B) inside a 32-wide fragment
-    const int lk = lane >> 5;   // which of the two k of an MFMA step
-
-    int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
-    const int m0 = tm * BM, n0 = tn * BN;
-    // two-level batch: z = outer * inner + inner_index (e.g. window x head)
-    const long long zo = blockIdx.y / g.inner, zi = blockIdx.y % g.inner;
-    const float* __restrict__ A = g.A + zo * g.sA2 + zi * g.sA;
-    const float* __restrict__ B = g.B + zo * g.sB2 + zi * g.sB;
-    const long long coff = zo * g.sC2 + zi * g.sC;
-
-    const int wm = (wave >> 1) * WM;
-    const int wn = (wave & 1) * WN;
-
-    // op(A) tile is BM x BK: rows m, cols k.  Stored (!TA) M x K -> tile (m, k);
-    // stored (TA) K x M -> tile (k, m).
-    TileRegs<TA ? BK : BM, TA ? BM : BK> ra;
-    // op(B) tile is BK x BN.  Stored (!TB) K x N -> tile (k, n); (TB) N x K -> tile (n, k).
-    TileRegs<TB ? BN : BK, TB ? BK : BN> rb;
-
-    // split-K: this workgroup reduces k in [kbeg, kend) (kchunk = K when unsplit)
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int kend = min(g.K, kbeg + g.kchunk);
-    auto gload = [&](int k0) {
-        if (TA) ra.load(A, g.lda, k0, m0, kend, M, g.vecA, tid);
-        else    ra.load(A, g.lda, m0, k0, M, kend, g.vecA, tid);
-        if (TB) rb.load(B, g.ldb, n0, k0, N, kend, g.vecB, tid);
-        else    rb.load(B, g.ldb, k0, n0, kend, N, g.vecB, tid);
-    };
-    auto lstore = [&](int buf) {
-        if (TA) ra.template store_direct<LDA>(As[buf], tid);
-        else    ra.template store_transposed<LDA>(As[buf], tid);
-        if (TB) rb.template store_transposed<LDB>(Bs[buf], tid);
-        else    rb.template store_direct<LDB>(Bs[buf], tid);
-    };
-
-    floatx16 acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-    if (nk > 0) {
-        gload(kbeg);
-        lstore(0);
-        __syncthreads();
-    }
-    for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        const bool more = kt + 1 < nk;
-        if (more) gload(kbeg + (kt + 1) * BK);
-        const float* as = As[cur];
-        const float* bs = Bs[cur];
-#pragma unroll
-        for (int kk = 0; kk < BK; kk += 2) {
-            float a[FM], b[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = as[(kk + lk) * LDA + wm + 32 * i + lr];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) b[j] = bs[(kk + lk) * LDB + wn + 32 * j + lr];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        if (more) lstore(cur ^ 1);
-        __syncthreads();
-    }
-
-    // Accumulator layout of a 32x32 block: element r of lane l sits at
-    // row 8*(r/4) + 4*(l/32) + r%4, column l%32.
-    if (g.splits > 1) {
-        // split-K partial of this slice: dense [split][batch][M][N], summed in
-        // slice order by splitk_reduce (a second launch: a device-scope fence
-        // inside this kernel would have to write back the per-XCD L2)
-        float* wz = g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) *
-                               (static_cast<long long>(M) * N);
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int col = n0 + wn + 32 * j + lr;
-                if (col >= N) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lk + (r & 3);
-                    if (row < M) wz[static_cast<long long>(row) * N + col] = acc[i][j][r];
-                }
-            }
-        return;
-    }
-    float* __restrict__ C = g.C + coff;
-    const float* R = g.R ? g.R + coff : C;
-    const int ldr = g.R ? g.ldr : g.ldc;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int col = n0 + wn + 32 * j + lr;
-            if (col >= N) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (row < M) {
-                    const float v = g.alpha * acc[i][j][r];
-                    C[static_cast<long long>(row) * g.ldc + col] =
-                        (g.beta != 0.f) ? v + g.beta * R[static_cast<long long>(row) * ldr + col] : v;
-                }
-            }
-        }
-}
-
-// sgemm_mfma_kernel with KS wave sets per workgroup (KS * 256 threads): set
-// s takes the K chunks s, s+KS, ... with its own double-buffered LDS, so each
-// SIMD holds KS waves and each set's chain of dependent chunk loads is KS
-// times shorter; the sets' partial tiles meet in LDS (fixed order).  For long
-// K on one or two 64x64 tiles per CU (1024^3: 29.1, 28.9-29.1 and 27.6-27.7 us
-// on one, four and two wave sets; split-K slices take four).  PF = 2: two
-// register sets per wave set, so chunk kt + 2 KS is in flight while chunk kt
-// runs and chunk kt + KS goes to LDS.
-template <int BM, int BN, int BK, bool TA, bool TB, int KS, int PF = 1, bool FULL = false>
-__global__ void __launch_bounds__(kThreads * KS)
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(2 * kThreads)
 sgemm_mfma_ks_kernel(const GemmArgs g)
 {
+    constexpr int BM = kKsTile, BN = kKsTile, BK = kKsK, KS = 2;
     constexpr int WM = BM / 2, WN = BN / 2;
-    constexpr int FM = WM / 32, FN = WN / 32;
     constexpr int LDA = TA ? BM + 4 : BM + 1;
     constexpr int LDB = TB ? BN + 1 : BN + 4;
     __shared__ float As[KS][2][BK * LDA];
@@ -385,22 +190,13 @@ sgemm_mfma_ks_kernel(const GemmArgs g)
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
     TileRegs<TA ? BK : BM, TA ? BM : BK> ra, ra2;
     TileRegs<TB ? BN : BK, TB ? BK : BN> rb, rb2;
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int kend = min(g.K, kbeg + g.kchunk);
     auto gload_to = [&](auto& xa, auto& xb, int k0) {
-        if constexpr (FULL) {
-            // K is whole chunks; M and N are clamped (M % 4 == 0 when A is
-            // stored K-major, N % 4 == 0 when B is)
-            if (TA) xa.load_full(A, g.lda, k0, m0, kend, M, gt);
-            else    xa.load_full(A, g.lda, m0, k0, M, kend, gt);
-            if (TB) xb.load_full(B, g.ldb, n0, k0, N, kend, gt);
-            else    xb.load_full(B, g.ldb, k0, n0, kend, N, gt);
-        } else {
-            if (TA) xa.load(A, g.lda, k0, m0, kend, M, g.vecA, gt);
-            else    xa.load(A, g.lda, m0, k0, M, kend, g.vecA, gt);
-            if (TB) xb.load(B, g.ldb, n0, k0, N, kend, g.vecB, gt);
-            else    xb.load(B, g.ldb, k0, n0, kend, N, g.vecB, gt);
-        }
+        // K is whole chunks; M and N are clamped (M % 4 == 0 when A is stored
+        // K-major, N % 4 == 0 when B is)
+        if (TA) xa.load_full(A, g.lda, k0, m0, g.K, M, gt);
+        else    xa.load_full(A, g.lda, m0, k0, M, g.K, gt);
+        if (TB) xb.load_full(B, g.ldb, n0, k0, N, g.K, gt);
+        else    xb.load_full(B, g.ldb, k0, n0, g.K, N, gt);
     };
     auto lstore_from = [&](const auto& xa, const auto& xb, int buf) {
         if (TA) xa.template store_direct<LDA>(As[grp][buf], gt);
@@ -408,601 +204,71 @@ sgemm_mfma_ks_kernel(const GemmArgs g)
         if (TB) xb.template store_transposed<LDB>(Bs[grp][buf], gt);
         else    xb.template store_direct<LDB>(Bs[grp][buf], gt);
     };
-    auto gload = [&](int k0) { gload_to(ra, rb, k0); };
-    auto lstore = [&](int buf) { lstore_from(ra, rb, buf); };
-    floatx16 acc[FM][FN];
+    floatx16 acc;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    const int nk = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int nk = g.K / BK;
     const int iters = (nk + KS - 1) / KS;
     auto mma = [&](int cur) {
         const float* as = As[grp][cur];
         const float* bs = Bs[grp][cur];
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 2) {
-            float a[FM], b[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = as[(kk + lk) * LDA + wm + 32 * i + lr];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) b[j] = bs[(kk + lk) * LDB + wn + 32 * j + lr];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+            const float a = as[(kk + lk) * LDA + wm + lr], b = bs[(kk + lk) * LDB + wn + lr];
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
         }
     };
-    // FULL: every chunk load is unconditional (past the last chunk a set
-    // reloads the last one, which it never stores), so the wait before an LDS
-    // store counts only the loads of the chunk being stored; a set with no
-    // chunk stores and reads only its own LDS, and adds a zero tile
-    if (FULL) gload(kbeg + min(grp, nk - 1) * BK);
-    else if (grp < nk) gload(kbeg + grp * BK);
-    else { ra = decltype(ra){}; rb = decltype(rb){}; }
-    if constexpr (PF == 2) {
-        // two register sets: chunk kt + 2 KS is loaded while chunk kt runs its
-        // MFMAs and chunk kt + KS (loaded one iteration earlier) goes to LDS
-        if (FULL) gload_to(ra2, rb2, kbeg + min(grp + KS, nk - 1) * BK);
-        else if (grp + KS < nk) gload_to(ra2, rb2, kbeg + (grp + KS) * BK);
-        lstore(0);
+    gload_to(ra, rb, min(grp, nk - 1) * BK);
+    gload_to(ra2, rb2, min(grp + KS, nk - 1) * BK);
+    lstore_from(ra, rb, 0);
+    __syncthreads();
+    // the register sets are picked at compile time (a run-time choice between
+    // them would put both in scratch memory)
+    auto body = [&](int it, auto setc) {
+        constexpr int L = decltype(setc)::value;   // the set loaded; the other is stored
+        auto& la = L == 0 ? ra : ra2;
+        auto& lb = L == 0 ? rb : rb2;
+        const auto& sa = L == 0 ? ra2 : ra;
+        const auto& sb = L == 0 ? rb2 : rb;
+        const int cur = it & 1;
+        const int kt = it * KS + grp;
+        gload_to(la, lb, min(kt + 2 * KS, nk - 1) * BK);
+        if (kt < nk) mma(cur);
+        if (kt + KS < nk) lstore_from(sa, sb, cur ^ 1);
         __syncthreads();
-        // the register sets are picked at compile time (a run-time choice
-        // between them would put both in scratch memory)
-        auto body = [&](int it, auto setc) {
-            constexpr int L = decltype(setc)::value;   // the set loaded; the other is stored
-            auto& la = L == 0 ? ra : ra2;
-            auto& lb = L == 0 ? rb : rb2;
-            const auto& sa = L == 0 ? ra2 : ra;
-            const auto& sb = L == 0 ? rb2 : rb;
-            const int cur = it & 1;
-            const int kt = it * KS + grp;
-            if (FULL) gload_to(la, lb, kbeg + min(kt + 2 * KS, nk - 1) * BK);
-            else if (kt + 2 * KS < nk) gload_to(la, lb, kbeg + (kt + 2 * KS) * BK);
-            if (kt < nk) mma(cur);
-            if (kt + KS < nk) lstore_from(sa, sb, cur ^ 1);
-            __syncthreads();
-        };
-        // FULL: no branch around the second body (past the last iteration it
-        // only reloads the last chunk; its MFMAs and LDS store are skipped),
-        // so every path through the loop has the same loads in flight and each
-        // LDS store waits for its own chunk alone; behind the branch the
-        // compiler made the stores wait for the next chunk's loads as well
-        // (tied head 512x2000x128 NT 7.04 -> 6.88 us, 512x2048x1024 27.05 ->
-        // 26.71; a third register set, chunks three ahead, was 8-15% slower)
-        for (int it = 0; it < iters; it += 2) {
-            body(it, std::integral_constant<int, 0>{});
-            if (FULL || it + 1 < iters) body(it + 1, std::integral_constant<int, 1>{});
-        }
-    } else {
-        lstore(0);
-        __syncthreads();
-        for (int it = 0; it < iters; ++it) {
-            const int cur = it & 1;
-            const int kt = it * KS + grp;
-            const bool more = it + 1 < iters;
-            const bool next_in = kt + KS < nk;
-            if (FULL) gload(kbeg + min(kt + KS, nk - 1) * BK);
-            else if (more && next_in) gload(kbeg + (kt + KS) * BK);
-            if (kt < nk) mma(cur);
-            if (more && next_in) lstore(cur ^ 1);
-            __syncthreads();
-        }
+    };
+    // No branch around the second body (past the last iteration it only
+    // reloads the last chunk; its MFMAs and LDS store are skipped), so every
+    // path through the loop has the same loads in flight and each LDS store
+    // waits for its own chunk alone (tied head 7.04 -> 6.88 us).
+    for (int it = 0; it < iters; it += 2) {
+        body(it, std::integral_constant<int, 0>{});
+        body(it + 1, std::integral_constant<int, 1>{});
     }
-    constexpr int SZ = 4 * FM * FN * 1024;   // one set's partial tiles (floats)
-    static_assert(KS == 1 || (KS - 1) * SZ <= KS * 2 * BK * LDA, "reduction area");
-    float* red = &As[0][0][0];   // sets 1..KS-1 leave their partial tiles here
+    float* red = &As[0][0][0];   // set 1 leaves its partial tile here
+    static_assert(4096 <= KS * 2 * BK * LDA, "reduction area");
     if (grp > 0) {
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    red[(grp - 1) * SZ + ((wave * FM + i) * FN + j) * 1024 + r * 64 + lane] = acc[i][j][r];
+        for (int r = 0; r < 16; ++r) red[wave * 1024 + r * 64 + lane] = acc[r];
     }
     __syncthreads();
     if (grp > 0) return;
 #pragma unroll
-    for (int t = 1; t < KS; ++t)   // in set order
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    acc[i][j][r] += red[(t - 1) * SZ + ((wave * FM + i) * FN + j) * 1024 + r * 64 + lane];
+    for (int r = 0; r < 16; ++r) acc[r] += red[wave * 1024 + r * 64 + lane];
     // Accumulator layout of a 32x32 block: element r of lane l sits at
     // row 8*(r/4) + 4*(l/32) + r%4, column l%32.
-    if (g.splits > 1) {   // split-K partial of this slice, summed by splitk_reduce
-        float* wz = g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) *
-                               (static_cast<long long>(M) * N);
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int col = n0 + wn + 32 * j + lr;
-                if (col >= N) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lk + (r & 3);
-                    if (row < M) wz[static_cast<long long>(row) * N + col] = acc[i][j][r];
-                }
-            }
-        return;
-    }
     float* __restrict__ C = g.C + coff;
     const float* R = g.R ? g.R + coff : C;
     const int ldr = g.R ? g.ldr : g.ldc;
+    const int col = n0 + wn + lr;
+    if (col >= N) return;
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-            const int col = n0 + wn + 32 * j + lr;
-            if (col >= N) continue;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (row < M) {   // streamed out, not left dirty in L2 for the kernel's end
-                    const float v = g.alpha * acc[i][j][r];
-                    __builtin_nontemporal_store(
-                        (g.beta != 0.f) ? v + g.beta * R[static_cast<long long>(row) * ldr + col] : v,
-                        &C[static_cast<long long>(row) * g.ldc + col]);
-                }
-            }
-        }
-}
-
-// ---------------------------------------------------------------------------
-// Large problems (at least one 256x256 tile per CU): 256x256 output tiles,
-// four waves of 128x128 (16 v_mfma_f32_32x32x2f32 accumulators each, 256
-// AGPRs, one wave per SIMD), 32-deep K tiles double-buffered in LDS (128 KB).
-//
-// Both LDS tiles are k-contiguous: As[m][k], Bs[n][k], 32 floats (8 quads of
-// 4 k) per row, quad q of row r stored at quad position q ^ swz(r) with
-// swz(r) = (r ^ (r >> 3)) & 7.  For an 8-deep K step at k0, lane l (row or
-// column r = l%32 of a 32-block, half h = l/32) fetches op(A)[r][k0+4h ..
-// k0+4h+3] and op(B)[k0+4h .. +3][c] with one ds_read_b128 each; MFMA t of
-// the step multiplies element t of both, so its two k slots are k0+t and
-// k0+4+t and the four MFMAs cover k0 .. k0+7 once.  A wave thus reads 8 b128
-// per 64 MFMAs.  The swizzle maps any 8 rows 8m .. 8m+7 (one 8-lane phase of
-// those reads) and any 8 rows 32m + 4j + c, j = 0..7 (a phase of the
-// transposed writes below) to 8 distinct quad positions: both are free of
-// bank conflicts.
-//
-// Global -> LDS, float4 loads along the stored contiguous dimension:
-//  - operand stored k-contiguous (A when !TA, B when TB): 8 lanes read one
-//    row's 32 k, written as they are (ds_write_b128);
-//  - operand stored K-major (A when TA, B when !TB): a lane reads a 4 k x 4
-//    column block (4 float4 from 4 k-rows, 64 lanes = 1 KB of a row per
-//    instruction) and writes it transposed: column c's 4 k as one b128.
-__device__ __forceinline__ float f4get(const float4& v, int t)
-{
-    return t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;   // t is a compile-time constant after unrolling
-}
-
-constexpr int kBig = 256;
-constexpr int kBigK = 32;
-constexpr int kLd256 = kBigK;        // floats per LDS row (quad-swizzled, no padding)
-constexpr int kBigQ = kBigK / 4;     // k quads per row of a tile
-constexpr int kBigLds = kBig * kLd256;
-
-__device__ __forceinline__ int big_swz(int row) { return (row ^ (row >> 3)) & 7; }
-
-template <bool KMAJOR, bool FULL, int ROWS = kBig>
-struct BigTileRegs {
-    // ROWS rows (m or n) x kBigK k of one operand: NS float4 per thread
-    static constexpr int NS = ROWS * kBigK / 4 / kThreads;
-    static constexpr int CQ = ROWS / 4;              // KMAJOR: column quads of a k row
-    static constexpr int KQS = kThreads / CQ;        // KMAJOR: k quads per slot block
-    static_assert(NS % 4 == 0 && kThreads % CQ == 0, "tile rows");
-    float4 v[NS];
-
-    // stored: element (row, k) at X[row * ld + k] (!KMAJOR) or X[k * ld + row] (KMAJOR).
-    // Slot s (0 .. NS-1) is one float4 load:
-    // !KMAJOR: row tid/8 + 32s, k quad tid%8;
-    // KMAJOR: k row 4kq + s%4 of block (columns 4(tid%CQ) .. +3, k quad kq = tid/CQ + KQS(s/4)).
-    // The slots are loaded and stored one at a time so that the main loop can
-    // spread them between MFMA groups; a KMAJOR store slot needs the four
-    // load slots of its block.
-    __device__ __forceinline__ void load_slot(int s, const float* __restrict__ X, int ld, int r0, int k0, int rmax,
-                                              int kmax, bool vec, int tid)
-    {
-        int gr, gk;
-        const float* src;
-        if (!KMAJOR) {
-            gr = r0 + tid / kBigQ + (kThreads / kBigQ) * s;
-            gk = k0 + 4 * (tid % kBigQ);
-            src = X + static_cast<long long>(gr) * ld + gk;
-        } else {
-            gr = r0 + 4 * (tid % CQ);
-            gk = k0 + 4 * (tid / CQ + KQS * (s >> 2)) + (s & 3);
-            src = X + static_cast<long long>(gk) * ld + gr;
-        }
-        // the 4 contiguous elements: (row gr, k gk..gk+3) or (k gk, columns gr..gr+3)
-        const int lim = KMAJOR ? rmax - gr : kmax - gk;
-        const bool lineok = KMAJOR ? gk < kmax : gr < rmax;
-        if (FULL || (vec && lineok && lim >= 4)) {
-            const float4 t = *reinterpret_cast<const float4*>(src);
-            v[s].x = t.x; v[s].y = t.y; v[s].z = t.z; v[s].w = t.w;   // per component: stays in VGPRs
-        } else {
-            v[s].x = (lineok && lim > 0) ? src[0] : 0.f;
-            v[s].y = (lineok && lim > 1) ? src[1] : 0.f;
-            v[s].z = (lineok && lim > 2) ? src[2] : 0.f;
-            v[s].w = (lineok && lim > 3) ? src[3] : 0.f;
-        }
-    }
-
-    __device__ __forceinline__ void store_slot(int s, float* lds, int tid) const
-    {
-        if (!KMAJOR) {
-            const int row = tid / kBigQ + (kThreads / kBigQ) * s;
-            *reinterpret_cast<float4*>(lds + row * kLd256 + 4 * ((tid % kBigQ) ^ big_swz(row))) = v[s];
-        } else {
-            // column 4(tid%CQ) + s%4 of block s/4: its four k from the block's four loads
-            const int b = s >> 2, c = s & 3;
-            const int row = 4 * (tid % CQ) + c;
-            const int kq = tid / CQ + KQS * b;
-            const float4 t = make_float4(f4get(v[4 * b + 0], c), f4get(v[4 * b + 1], c), f4get(v[4 * b + 2], c),
-                                         f4get(v[4 * b + 3], c));
-            *reinterpret_cast<float4*>(lds + row * kLd256 + 4 * (kq ^ big_swz(row))) = t;
-        }
-    }
-};
-
-// FULL: M and N multiples of TILE, K of kBigK, k-contiguous operands 16-byte
-// aligned -- every tile load is in bounds and unconditional.  TILE = 128 is
-// the same kernel on 128x128 tiles (four waves of 64x64, 4 accumulators each,
-// 64 KB of LDS: two workgroups per CU), for problems with fewer 256x256 tiles
-// than CUs but many 128x128 ones.
-template <bool TA, bool TB, bool FULL, int TILE = kBig>
-__global__ void __launch_bounds__(kThreads)
-sgemm_256_kernel(const GemmArgs g)
-{
-    constexpr int F = TILE / 64;   // 32x32 blocks per wave and dimension
-    constexpr int LDS = TILE * kLd256;
-    __shared__ float As[2][LDS];
-    __shared__ float Bs[2][LDS];
-    const int M = g.M, N = g.N;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int lr = lane & 31;
-    const int h = lane >> 5;
-    int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
-    const int m0 = tm * TILE, n0 = tn * TILE;
-    const long long zo = blockIdx.y / g.inner, zi = blockIdx.y % g.inner;
-    // split-K: this workgroup takes k in [kbeg, kbeg + K); the operands are
-    // offset to the slice start (k runs along a stored row of A when !TA and
-    // of B when TB, down the stored columns otherwise)
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int K = min(g.K, kbeg + g.kchunk) - kbeg;
-    const float* __restrict__ A = g.A + zo * g.sA2 + zi * g.sA + (TA ? static_cast<long long>(kbeg) * g.lda : kbeg);
-    const float* __restrict__ B = g.B + zo * g.sB2 + zi * g.sB + (TB ? kbeg : static_cast<long long>(kbeg) * g.ldb);
-    const long long coff = zo * g.sC2 + zi * g.sC;
-    const int wm = (wave >> 1) * (TILE / 2), wn = (wave & 1) * (TILE / 2);
-
-    BigTileRegs<TA, FULL, TILE> ra;    // op(A): row m; stored M x K (!TA) or K x M (TA)
-    BigTileRegs<!TB, FULL, TILE> rb;   // op(B): row n; stored N x K (TB) or K x N (!TB)
-    constexpr int NS = BigTileRegs<TA, FULL, TILE>::NS;
-    auto gload = [&](int s, int k0) {
-        ra.load_slot(s, A, g.lda, m0, k0, M, K, g.vecA, tid);
-        rb.load_slot(s, B, g.ldb, n0, k0, N, K, g.vecB, tid);
-    };
-    auto lstore = [&](int s, int buf) {
-        ra.store_slot(s, As[buf], tid);
-        rb.store_slot(s, Bs[buf], tid);
-    };
-
-    floatx16 acc[F][F];
-#pragma unroll
-    for (int i = 0; i < F; ++i)
-#pragma unroll
-        for (int j = 0; j < F; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    // Fragments of one 8-deep step: a[i] = op(A) rows wm+32i+lr, b[j] = op(B)
-    // columns wn+32j+lr, k = k0+4h .. k0+4h+3 each.
-    // Quad k0/4 + h of row wm + 32i + lr sits at position (k0/4 + h) ^ swz, with
-    // swz = (lr ^ (lr >> 3) ^ 4(i & 1)) & 7 (wm, wn are multiples of 64);
-    // k0/4 is even, so the position is (k0/4) ^ g with g = h ^ swz.
-    struct Frag { float4 a[F], b[F]; };
-    const int g_even = (h ^ lr ^ (lr >> 3)) & 7;
-    auto read_frag = [&](Frag& f, int buf, int k0) {
-        const float* as = As[buf] + (wm + lr) * kLd256;
-        const float* bs = Bs[buf] + (wn + lr) * kLd256;
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-            f.a[i] = *reinterpret_cast<const float4*>(as + 32 * i * kLd256 + 4 * ((k0 / 4) ^ g_even ^ (4 * (i & 1))));
-#pragma unroll
-        for (int j = 0; j < F; ++j)
-            f.b[j] = *reinterpret_cast<const float4*>(bs + 32 * j * kLd256 + 4 * ((k0 / 4) ^ g_even ^ (4 * (j & 1))));
-    };
-    auto mma_t = [&](const Frag& f, int t) {
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(f4get(f.a[i], t), f4get(f.b[j], t), acc[i][j],
-                                                                0, 0, 0);
-    };
-
-    // Software pipeline over the four 8-deep steps of a K tile:
-    //   steps 0-2: read the next step's fragments, then four groups of F*F
-    //     MFMAs; after each group, steps 0-1 issue one slot of the next tile's
-    //     global loads (8 slots; with TILE = 128, 4 slots in step 0), step 2
-    //     writes two slots (one) to the other LDS buffer (so the loads have
-    //     had two steps to land);
-    //   barrier; read the next tile's step-0 fragments; step 3's MFMAs.
-    // Spreading the loads and LDS writes keeps the MFMA pipe fed (a CU's
-    // address path takes 64 B/clk: a whole tile's 64 KB issued at once stalls
-    // the waves for ~1K cycles).  All reads of an LDS buffer are issued before
-    // the barrier that precedes its next write.
-    constexpr int kSteps = kBigK / 8;
-    static_assert(kSteps == 4 && kBigQ == 8 && (NS == 8 || NS == 4), "the load/store schedule assumes 32-deep K tiles");
-    const int nk = (K + kBigK - 1) / kBigK;
-    Frag f[2];
-    if (nk > 0) {
-#pragma unroll
-        for (int sl = 0; sl < NS; ++sl) gload(sl, 0);
-#pragma unroll
-        for (int sl = 0; sl < NS; ++sl) lstore(sl, 0);
-        __syncthreads();
-        read_frag(f[0], 0, 0);
-    }
-    // The loads, stores and reads of the next tile are unconditional (no
-    // branches for the waitcnt placement to be conservative about): on the
-    // last tile they repeat the current tile's loads into the idle buffer.
-    for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        const int kn = (kt + 1 < nk ? kt + 1 : kt) * kBigK;
-#pragma unroll
-        for (int st = 0; st + 1 < kSteps; ++st) {
-            read_frag(f[(st + 1) & 1], cur, 8 * (st + 1));
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                __builtin_amdgcn_sched_barrier(0);
-                mma_t(f[st & 1], t);
-                __builtin_amdgcn_sched_barrier(0);
-                if (NS == 8) {
-                    if (st < 2) {
-                        gload(4 * st + t, kn);
-                    } else {
-                        lstore(2 * t, cur ^ 1);
-                        lstore(2 * t + 1, cur ^ 1);
-                    }
-                } else {
-                    if (st == 0) gload(t, kn);
-                    else if (st == 2) lstore(t, cur ^ 1);
-                }
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();
-        read_frag(f[0], cur ^ 1, 0);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            __builtin_amdgcn_sched_barrier(0);
-            mma_t(f[1], t);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-
-    if (g.splits > 1) {
-        // raw slice sums, [slice][batch][M][N]; the ordered reduce applies
-        // alpha, beta and R
-        float* __restrict__ wz =
-            g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * (static_cast<long long>(M) * N);
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j) {
-                const int col = n0 + wn + 32 * j + lr;
-                if (!FULL && col >= N) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (FULL || row < M) wz[static_cast<long long>(row) * N + col] = acc[i][j][r];
-                }
-            }
-        return;
-    }
-    float* __restrict__ C = g.C + coff;
-    const float* R = g.R ? g.R + coff : C;
-    const int ldr = g.R ? g.ldr : g.ldc;
-    // The beta test sits outside the unrolled stores (one branch, not 256).
-    auto epilogue = [&](auto use_rc) {
-        constexpr bool USE_R = decltype(use_rc)::value;
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j) {
-                const int col = n0 + wn + 32 * j + lr;
-                if (!FULL && col >= N) continue;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                    if (FULL || row < M) {
-                        float v = g.alpha * acc[i][j][r];
-                        if (USE_R) v += g.beta * R[static_cast<long long>(row) * ldr + col];
-                        C[static_cast<long long>(row) * g.ldc + col] = v;
-                    }
-                }
-            }
-    };
-    if (g.beta != 0.f) epilogue(std::true_type{});
-    else epilogue(std::false_type{});
-}
-
-int launch_reduce(const GemmArgs& g, int batch, hipStream_t stream);
-
-template <int TILE>
-int launch_big(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
-{
-    g.tiles_m = ceil_div(g.M, TILE);
-    g.tiles_n = ceil_div(g.N, TILE);
-    const long long nwg = static_cast<long long>(g.tiles_m) * g.tiles_n;
-    if (nwg > 0x7fffffffLL) return fail(LHIP_E_CAPACITY, "sgemm: %lld workgroups exceed the grid limit", nwg);
-    if (g.splits <= 1 || !g.ws) { g.splits = 1; g.kchunk = g.K; g.ws = nullptr; }
-    dim3 grid(static_cast<unsigned>(nwg), batch, g.splits), block(kThreads, 1, 1);
-    // FULL: every tile and every K slice whole (slices start at multiples of
-    // kchunk, itself a multiple of the 32-deep K tile)
-    const bool full = g.M % TILE == 0 && g.N % TILE == 0 && g.K % kBigK == 0 && g.kchunk % kBigK == 0 &&
-                      (ta || g.vecA) && (!tb || g.vecB);
-    auto go = [&](auto fullc) {
-        constexpr bool F = decltype(fullc)::value;
-        if (!ta && !tb) klaunch(sgemm_256_kernel<false, false, F, TILE>, grid, block, 0, stream, g);
-        else if (ta && !tb) klaunch(sgemm_256_kernel<true, false, F, TILE>, grid, block, 0, stream, g);
-        else if (!ta && tb) klaunch(sgemm_256_kernel<false, true, F, TILE>, grid, block, 0, stream, g);
-        else klaunch(sgemm_256_kernel<true, true, F, TILE>, grid, block, 0, stream, g);
-    };
-    if (full) go(std::true_type{});
-    else go(std::false_type{});
-    const int rc = check_launch("sgemm (256): kernel launch");
-    if (rc != LHIP_OK || g.splits <= 1) return rc;
-    return launch_reduce(g, batch, stream);
-}
-
-int launch_256(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
-{
-    return launch_big<kBig>(ta, tb, g, batch, stream);
-}
-
-// ---------------------------------------------------------------------------
-// Small problems (fewer 64x64 output tiles than CUs, e.g. every GEMM of the
-// C2 LMTrain step): one workgroup per 32x32 output tile, and the NW waves of
-// the workgroup (4, or 8 once K >= 256) split K among themselves -- wave w
-// takes the 8-deep K steps w, w+NW, w+2NW, ... -- each accumulating the whole
-// 32x32 tile, so one tile's K loop runs on all four SIMDs of its CU.  The
-// partial tiles are summed in LDS in wave order (deterministic).  Operands are loaded straight from
-// global memory into MFMA fragments: for an 8-deep K step, lane l (row or
-// column l%32, half h = l/32) holds op(A)[row][k0+4h .. k0+4h+3] and
-// op(B)[k0+4h .. k0+4h+3][col]; MFMA i of the step multiplies element i of
-// both, so the two halves of one v_mfma_f32_32x32x2f32 cover k0+i and
-// k0+4+i and the four MFMAs cover k0 .. k0+7 exactly once.  The contiguous
-// operand dimension is read as float4 when aligned, otherwise element-wise.
-//
-// With BR (batch-reduce, non-transposed A only) the K range is kblocks blocks
-// of Kb (Kb % 4 == 0): logical k lies in block j = k / Kb, whose operands start
-// at A + j*sAk and B + j*sBk, so C = alpha * sum_j A_j . op(B_j) + beta * R in
-// one launch.  A lane's four k never straddle a block.
-template <bool TA, bool TB, bool BR, int NW>
-__global__ void __launch_bounds__(64 * NW)
-sgemm_small_kernel(const GemmArgs g)
-{
-    __shared__ float red[NW][16][64];
-    const int M = g.M, N = g.N;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int lr = lane & 31;
-    const int h = lane >> 5;
-    int tm, tn;
-    xcd_tile(blockIdx.x, gridDim.x, g.tiles_n, tm, tn);
-    const int m0 = tm * 32, n0 = tn * 32;
-    const long long zo = blockIdx.y / g.inner, zi = blockIdx.y % g.inner;
-    const float* __restrict__ A = g.A + zo * g.sA2 + zi * g.sA;
-    const float* __restrict__ B = g.B + zo * g.sB2 + zi * g.sB;
-    const long long coff = zo * g.sC2 + zi * g.sC;
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int kend = min(g.K, kbeg + g.kchunk);
-    const int row = m0 + lr;      // this lane's A row
-    const int col = n0 + lr;      // this lane's B column
-    const bool rok = row < M, cok = col < N;
-
-    floatx16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-
-    // Each pass issues the loads of kSmallU K steps before any of their MFMAs,
-    // so that many loads are in flight per wave (these launches have few
-    // workgroups: latency, not bandwidth, bounds them).
-    constexpr int U = kSmallU;
-    for (int kp = kbeg + 8 * wave; kp < kend; kp += 8 * NW * U) {
-        float a[U][4], b[U][4];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int kl = kp + 8 * NW * u + 4 * h;   // first of this lane's four k (logical)
-            const bool kfull = kl + 3 < kend;
-            const int kend_l = kend - kl;         // valid k from kl on: i < kend_l
-            int kb = kl;
-            const float* __restrict__ Ab = A;
-            const float* __restrict__ Bb = B;
-            if (BR) {
-                const int j = kl / g.Kb;
-                kb = kl - j * g.Kb;
-                Ab = A + j * g.sAk;
-                Bb = B + j * g.sBk;
-            }
-            if (!TA) {
-                const float* src = Ab + static_cast<long long>(row) * g.lda + kb;
-                if (g.vecA && rok && kfull) {
-                    const float4 v = *reinterpret_cast<const float4*>(src);
-                    a[u][0] = v.x; a[u][1] = v.y; a[u][2] = v.z; a[u][3] = v.w;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) a[u][i] = (rok && i < kend_l) ? src[i] : 0.f;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    a[u][i] = (rok && i < kend_l) ? Ab[static_cast<long long>(kb + i) * g.lda + row] : 0.f;
-            }
-            if (!TB) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    b[u][i] = (cok && i < kend_l) ? Bb[static_cast<long long>(kb + i) * g.ldb + col] : 0.f;
-            } else {
-                const float* src = Bb + static_cast<long long>(col) * g.ldb + kb;
-                if (g.vecB && cok && kfull) {
-                    const float4 v = *reinterpret_cast<const float4*>(src);
-                    b[u][0] = v.x; b[u][1] = v.y; b[u][2] = v.z; b[u][3] = v.w;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) b[u][i] = (cok && i < kend_l) ? src[i] : 0.f;
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][i], b[u][i], acc, 0, 0, 0);
-    }
-
-    // sum the waves' tiles in wave order; thread (wave w, lane l) finishes
-    // accumulator registers (16/NW)w .. (16/NW)(w+1)-1 of lane l
-#pragma unroll
-    for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[r];
-    __syncthreads();
-    const int ocol = n0 + (lane & 31);
-    const int lk = lane >> 5;
-    float* wz = nullptr;
-    if (g.splits > 1)
-        wz = g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * (static_cast<long long>(M) * N);
-    float* __restrict__ C = g.C + coff;
-    const float* R = g.R ? g.R + coff : C;
-    const int ldr = g.R ? g.ldr : g.ldc;
-    constexpr int RPW = 16 / NW;
-#pragma unroll
-    for (int q = 0; q < RPW; ++q) {
-        const int r = RPW * wave + q;
-        float v = red[0][r][lane];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) v += red[w][r][lane];
-        const int orow = m0 + 8 * (r >> 2) + 4 * lk + (r & 3);
-        if (orow >= M || ocol >= N) continue;
-        if (wz) {
-            wz[static_cast<long long>(orow) * N + ocol] = v;
-        } else {
-            const float o = g.alpha * v;
-            C[static_cast<long long>(orow) * g.ldc + ocol] =
-                (g.beta != 0.f) ? o + g.beta * R[static_cast<long long>(orow) * ldr + ocol] : o;
+    for (int r = 0; r < 16; ++r) {
+        const int row = m0 + wm + 8 * (r >> 2) + 4 * lk + (r & 3);
+        if (row < M) {   // streamed out, not left dirty in L2 for the kernel's end
+            const float v = g.alpha * acc[r];
+            __builtin_nontemporal_store((g.beta != 0.f) ? v + g.beta * R[static_cast<long long>(row) * ldr + col] : v,
+                                        &C[static_cast<long long>(row) * g.ldc + col]);
         }
     }
 }
@@ -1019,7 +285,7 @@ sgemm_small_kernel(const GemmArgs g)
 // Waves 1..3 hand their sums to wave 0 through LDS, added in wave order.  A K
 // split over blockIdx.y writes [split][M][N] partials that splitk_reduce adds
 // in split order.
-constexpr int kSkinnyMax = 64;
+constexpr int kSkinnyMax = 32;
 constexpr int kSkinnyCols = 256;    // columns per workgroup (64 lanes x float4)
 constexpr int kSkinnyKC = 256;      // K rows of A staged per chunk
 
@@ -1628,20 +894,6 @@ sgemm_tiny_kernel(const GemmArgs g)
 }
 
 // Eight waves share K once it is long enough for each to get a full pass.
-constexpr int kSmallWavesLongK = 8;
-inline bool small_long_k(const GemmArgs& g) { return g.kchunk >= 8 * 4 * kSmallU; }
-
-template <bool TA, bool TB, bool BR>
-void launch_small_t(const GemmArgs& g, dim3 grid, hipStream_t stream)
-{
-    if (small_long_k(g))
-        klaunch(sgemm_small_kernel<TA, TB, BR, kSmallWavesLongK>, grid, dim3(64 * kSmallWavesLongK), 0, stream, g);
-    else
-        klaunch(sgemm_small_kernel<TA, TB, BR, 4>, grid, dim3(256), 0, stream, g);
-}
-
-int launch_reduce(const GemmArgs& g, int batch, hipStream_t stream);
-
 // PIPE: K needs more than one pass of the four waves (64 * kSmallU deep)
 template <bool PIPE, int NW>
 void launch_tiny_t(int ta, int tb, const GemmArgs& g, dim3 grid, hipStream_t stream)
@@ -1674,26 +926,6 @@ int launch_tiny(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
     return launch_reduce(g, batch, stream);
 }
 
-int launch_small(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
-{
-    g.tiles_m = ceil_div(g.M, 32);
-    g.tiles_n = ceil_div(g.N, 32);
-    const long long nwg = static_cast<long long>(g.tiles_m) * g.tiles_n;
-    if (nwg > 0x7fffffffLL) return fail(LHIP_E_CAPACITY, "sgemm: %lld workgroups exceed the grid limit", nwg);
-    if (g.splits <= 1) { g.splits = 1; g.kchunk = g.K; g.ws = nullptr; }
-    dim3 grid(static_cast<unsigned>(nwg), batch, g.splits);
-    if (g.Kb != g.K) {   // batch-reduce (sgemm_run admits it for non-transposed A only)
-        if (!tb) launch_small_t<false, false, true>(g, grid, stream);
-        else launch_small_t<false, true, true>(g, grid, stream);
-    } else if (!ta && !tb) launch_small_t<false, false, false>(g, grid, stream);
-    else if (ta && !tb) launch_small_t<true, false, false>(g, grid, stream);
-    else if (!ta && tb) launch_small_t<false, true, false>(g, grid, stream);
-    else launch_small_t<true, true, false>(g, grid, stream);
-    int rc = check_launch("sgemm (small): kernel launch");
-    if (rc != LHIP_OK || g.splits <= 1 || g.skip_reduce) return rc;
-    return launch_reduce(g, batch, stream);
-}
-
 // Skinny path: M <= 64, B not transposed, one product (no batch, no
 // batch-reduce), at least one full wave of columns.
 bool skinny_ok(int ta, int tb, int m, int n, int batch, int kblocks)
@@ -1702,32 +934,10 @@ bool skinny_ok(int ta, int tb, int m, int n, int batch, int kblocks)
     return !tb && m >= 1 && m <= kSkinnyMax && n >= kSkinnyCols && batch == 1 && kblocks == 1;
 }
 
-// 33..64 rows with long K and wide N: one 64-row tile band of 64x64 tiles on
-// four wave sets, split over K so that tiles x slices fill the CUs (M = 64,
-// K = N = 4096: 64 tiles x 4 slices, 31.8 us against 45 us on the skinny MFMA
-// form and its reduce).
-bool ks_split_ok(int m, int n, int k, int batch)
-{
-    return batch == 1 && m > 32 && m <= 64 && n >= 1024 && k >= 2048;
-}
-
-int ks_split_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
-{
-    const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    const long long tiles = ceil_div(n, 64);
-    long long s = std::max<long long>(1, cus / tiles);
-    s = std::min<long long>(s, k / 512);
-    s = std::min<long long>(s, 16);
-    const long long mn = static_cast<long long>(m) * n;
-    s = std::min<long long>(s, static_cast<long long>(ws_floats / mn));
-    if (s < 2) return 1;
-    const int kchunk = ceil_div(ceil_div(k, static_cast<int>(s)), 32) * 32;
-    *kchunk_out = kchunk;
-    return ceil_div(k, kchunk);
-}
-
 // Rows of C up to which the VALU form is used; 3..64 rows take the MFMA form.
 constexpr int kSkinnyValuMax = 2;
+
+}  // namespace
 
 // K slices of the skinny path: about two workgroups per CU, at least 64 K rows
 // per workgroup, and partials (written, then read back by the reduce) at most
@@ -1754,6 +964,8 @@ int skinny_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
     *kchunk_out = kchunk;
     return ceil_div(k, kchunk);
 }
+
+namespace {
 
 template <bool TA, bool VEC>
 void launch_skinny_t(const GemmArgs& g, dim3 grid, hipStream_t stream)
@@ -1785,72 +997,41 @@ int launch_skinny(int ta, GemmArgs g, hipStream_t stream)
                 else klaunch(sgemm_skinny_mfma_lds_kernel<false, false, MG>, grid, T, 0, stream, g);
             }
         };
-        const int mg = ceil_div(g.M, 16);
-        if (mg == 1) go(std::integral_constant<int, 1>{});
-        else if (mg == 2) go(std::integral_constant<int, 2>{});
-        else if (mg == 3) go(std::integral_constant<int, 3>{});
-        else go(std::integral_constant<int, 4>{});
+        if (g.M <= 16) go(std::integral_constant<int, 1>{});
+        else go(std::integral_constant<int, 2>{});
     }
     int rc = check_launch("sgemm (skinny): kernel launch");
     if (rc != LHIP_OK || g.splits <= 1) return rc;
     return launch_reduce(g, 1, stream);
 }
 
-template <int BM, int BN, int BK, int KS>
-int launch_cfg_ks(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
+// One 64x64 tile per CU at most, whole 32-deep chunks of a short K and
+// operands whose rows take float4 loads: the fp32 cores and one load round trip
+// beat the conversion and the deeper pipeline of the three-term kernel (the C2
+// step's tied head, 512x2000x128: 6.1 us against 7.9; 64 batches of
+// 256x64x256: 11.3-12.4 us against 12.3-12.9; past K = 256 the three-term
+// kernel is faster: 2048x512x512 13.6 against 14.8).  M and N need not be whole tiles: rows and columns past them
+// are clamped into the operands.
+bool ks_best(int ta, int tb, int m, int n, int k, int batch, int vecA, int vecB)
 {
-    g.tiles_m = ceil_div(g.M, BM);
-    g.tiles_n = ceil_div(g.N, BN);
-    const long long nwg = static_cast<long long>(g.tiles_m) * g.tiles_n;
-    if (nwg > 0x7fffffffLL) return fail(LHIP_E_CAPACITY, "sgemm: %lld workgroups exceed the grid limit", nwg);
-    if (g.splits <= 1) { g.splits = 1; g.kchunk = g.K; g.ws = nullptr; }
-    dim3 grid(static_cast<unsigned>(nwg), batch, g.splits), block(KS * kThreads, 1, 1);
-    // NN (A's 32-deep chunk is 64 row segments of 128 bytes) loads two chunks
-    // ahead: 1024^3 32.3 -> 30.8 us and 2048x1024x512 31.9 -> 31.3 (medians of
-    // six alternating rounds on one box); TN and NT measured 0.4-0.5 us slower
-    // that way
-    // Whole chunks with float4-loadable operands: unconditional
-    // loads two chunks ahead (1024^3 NN 29.5 -> 26.6 us, NT 26.9 -> 24.2, TN
-    // 27.5 -> 26.0, 2048x1024x512 30.6 -> 25.8, the M = 64 band 29.4 -> 27.3;
-    // with the loads behind a branch each LDS store waited for every load in
-    // flight, the chunk two ahead included)
-    // (M and N need not be whole tiles: rows and columns past them are
-    // clamped into the operands; M % 4 == 0 when A is stored K-major and
-    // N % 4 == 0 when B is.  The tied head of the C2 step, 512x2000x128 NT,
-    // 7.2 -> 6.8 us; a 60x4000x4096 band 31.5 -> 27.8.)
-    const bool full = (!ta || g.M % 4 == 0) && (tb || g.N % 4 == 0) && g.K % BK == 0 && g.kchunk % BK == 0 &&
-                      g.vecA && g.vecB && g.Kb == g.K;
-    if (full) {
-        if (!ta && !tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, false, false, KS, 2, true>, grid, block, 0, stream, g);
-        else if (ta && !tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, true, false, KS, 2, true>, grid, block, 0, stream, g);
-        else if (!ta && tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, false, true, KS, 2, true>, grid, block, 0, stream, g);
-        else klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, true, true, KS, 2, true>, grid, block, 0, stream, g);
-    } else if (!ta && !tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, false, false, KS, 2>, grid, block, 0, stream, g);
-    else if (ta && !tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, true, false, KS>, grid, block, 0, stream, g);
-    else if (!ta && tb) klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, false, true, KS>, grid, block, 0, stream, g);
-    else klaunch(sgemm_mfma_ks_kernel<BM, BN, BK, true, true, KS>, grid, block, 0, stream, g);
-    int rc = check_launch("sgemm: kernel launch");
-    if (rc != LHIP_OK || g.splits <= 1 || g.skip_reduce) return rc;
-    return launch_reduce(g, batch, stream);
+    const int cus = st().cu_count > 0 ? st().cu_count : 256;
+    const long long tiles64 = static_cast<long long>(ceil_div(m, kKsTile)) * ceil_div(n, kKsTile) * batch;
+    return tiles64 <= cus && k <= 256 && k % kKsK == 0 && vecA && vecB && (!ta || m % 4 == 0) && (tb || n % 4 == 0);
 }
 
-template <int BM, int BN, int BK>
-int launch_cfg(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
+int launch_ks(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
 {
-    g.tiles_m = ceil_div(g.M, BM);
-    g.tiles_n = ceil_div(g.N, BN);
-    const long long nwg = static_cast<long long>(g.tiles_m) * g.tiles_n;
-    if (nwg > 0x7fffffffLL) return fail(LHIP_E_CAPACITY, "sgemm: %lld workgroups exceed the grid limit", nwg);
-    if (g.splits <= 1) { g.splits = 1; g.kchunk = g.K; g.ws = nullptr; }
-    dim3 grid(static_cast<unsigned>(nwg), batch, g.splits), block(kThreads, 1, 1);
-    if (!ta && !tb) klaunch(sgemm_mfma_kernel<BM, BN, BK, false, false>, grid, block, 0, stream, g);
-    else if (ta && !tb) klaunch(sgemm_mfma_kernel<BM, BN, BK, true, false>, grid, block, 0, stream, g);
-    else if (!ta && tb) klaunch(sgemm_mfma_kernel<BM, BN, BK, false, true>, grid, block, 0, stream, g);
-    else klaunch(sgemm_mfma_kernel<BM, BN, BK, true, true>, grid, block, 0, stream, g);
-    int rc = check_launch("sgemm: kernel launch");
-    if (rc != LHIP_OK || g.splits <= 1 || g.skip_reduce) return rc;
-    return launch_reduce(g, batch, stream);
+    g.tiles_m = ceil_div(g.M, kKsTile);
+    g.tiles_n = ceil_div(g.N, kKsTile);
+    const dim3 grid(static_cast<unsigned>(g.tiles_m) * g.tiles_n, batch, 1), block(2 * kThreads, 1, 1);
+    if (!ta && !tb) klaunch(sgemm_mfma_ks_kernel<false, false>, grid, block, 0, stream, g);
+    else if (ta && !tb) klaunch(sgemm_mfma_ks_kernel<true, false>, grid, block, 0, stream, g);
+    else if (!ta && tb) klaunch(sgemm_mfma_ks_kernel<false, true>, grid, block, 0, stream, g);
+    else klaunch(sgemm_mfma_ks_kernel<true, true>, grid, block, 0, stream, g);
+    return check_launch("sgemm: kernel launch");
 }
+
+}  // namespace
 
 int launch_reduce(const GemmArgs& g, int batch, hipStream_t stream)
 {
@@ -1871,6 +1052,8 @@ int launch_reduce(const GemmArgs& g, int batch, hipStream_t stream)
     klaunch(splitk_reduce, static_cast<int>(rg), 256, 0, stream, g, batch);
     return check_launch("sgemm: split-K reduce");
 }
+
+namespace {
 
 // Grouped transposed-A products (the weight gradients of the LMTrain step:
 // dW = X^T . dY with X, dY row-major over the same B*T rows, every layer's and
@@ -2449,136 +1632,45 @@ int sgemm_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream,
     return rmsnorm_bwd_colsum_multi(cs->partial, cs->nparts, cs->out, cs->njobs, cs->cols, cs->acc, stream);
 }
 
-// Below the 64x64-tile threshold, the 32x32 small kernel is used unless K is
-// long AND both output dimensions exceed 64: its 32-wide tiles re-read A N/32
-// times and B M/32 times, which for long K costs more L2/MALL traffic than
-// the 64x64 tiles (+ split-K) save in latency.
-bool use_small_kernel(int m, int n, int k) { return k <= 2048 || m <= 64 || n <= 64; }
-
-
-// 256x256 tiles split over K (one batch): when the tiles alone would fill
-// between a quarter and all of the CUs (e.g. 2048^3: 64 tiles), each tile's K
-// is cut into slices of at least 512 so that tiles x slices covers the CUs;
-// the slices are summed in order by the reduce.  K % 32 == 0 keeps every
-// slice whole.  Returns the slice count (1: not this path).
-int split256_plan(int m, int n, int k, int batch, size_t ws_floats, int* kchunk_out)
+// 16x16 tiles whose consumer sums the slices itself (no reduce launch): one
+// software pass per slice, slices a multiple of 64 deep.
+int tiny_unreduced_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
 {
-    const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    const long long tiles = static_cast<long long>(ceil_div(m, kBig)) * ceil_div(n, kBig);
-    if (batch != 1 || tiles >= cus || 4 * tiles < cus || k % kBigK != 0) return 1;
-    long long s = (cus + tiles - 1) / tiles;
-    s = std::min<long long>(s, k / 512);
-    const long long mn = static_cast<long long>(m) * n;
-    if (mn > 0) s = std::min<long long>(s, static_cast<long long>(ws_floats / mn));
+    constexpr int pass = 64 * kSmallU;
+    if (k <= pass) return 1;
+    long long s = std::min<long long>(ceil_div(k, pass), 64);
+    s = std::min<long long>(s, static_cast<long long>(ws_floats / (static_cast<size_t>(m) * n)));
     if (s < 2) return 1;
-    const int kchunk = ceil_div(ceil_div(k, static_cast<int>(s)), kBigK) * kBigK;
-    const int splits = ceil_div(k, kchunk);
-    if (splits < 2) return 1;
+    const int kchunk = ceil_div(ceil_div(k, static_cast<int>(s)), 64) * 64;
     *kchunk_out = kchunk;
-    return splits;
+    return ceil_div(k, kchunk);
 }
 
-// The 256x256-tile kernel on 128x128 tiles: when there are fewer 256x256
-// tiles than CUs but at least ~3/4 of a CU's worth of 128x128 tiles, unless
-// the 256x256 tiles split over K into slices of 1024 or more (long K: the
-// big tiles' 84% beat the small ones' 79% at 2048x2048x8192).  Measured:
-// 2048^3 151.8 (256x256 in 4 slices of 512) -> 143.1 us; the C3 logits
-// 512x32000x128 57.3 -> 51.0 us; C3 dW 128x32000x512 52.4 -> 45.7 us.
-// Few 128x128 tiles (at most an eighth of the CUs) over a long K: the same
-// kernel split over K into one slice per CU's worth of tiles, slices of 448+
-// (C3 dhidden 512x128x32000: 4 tiles x 64 slices of 512, 53-57 -> 48 us; a
-// split count that leaves CUs idle or doubles up measured slower).  Batch 1.
-int big128_split_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
+// Products with fewer 32x32 tiles than CUs that stay on 16x16 tiles: four
+// times the workgroups, and up to K = 512 one round trip of loads.  K up to
+// 1024; up to 2048 when both operands take float4 loads (256x256x1536 NT 11.1
+// us against 12.1 on the three-term kernel, 512x128x2000 10.2 against 11.6;
+// unaligned 238x474x1199 28.4 against 12.4); up to 4096 where B is read along
+// its rows and the product is one column tile wide, or A is K-major
+// (4096x16x4096 NN 21.2 against 25.0, TN 23.2 against 31.0; 128x128x4096 TN
+// 10.8 against 12.8; but 16x4096x4096 NT 38.4 against 23.8).
+bool tiny_best(int ta, int tb, int m, int n, int k, int batch, int vecA, int vecB)
 {
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    if (m <= 64 || n <= 64) return 1;
-    const long long t128 = static_cast<long long>(ceil_div(m, 128)) * ceil_div(n, 128);
-    if (8 * t128 > cus) return 1;
-    const long long s = cus / t128;
-    const int kchunk = static_cast<int>(ceil_div(ceil_div(static_cast<long long>(k), s), 32LL) * 32);
-    if (kchunk < 448) return 1;
-    const int splits = ceil_div(k, kchunk);
-    if (splits < 2 || static_cast<size_t>(splits) * m * n > ws_floats) return 1;
-    *kchunk_out = kchunk;
-    return splits;
-}
-
-bool big128_ok(int m, int n, int batch, int s256, int kc256)
-{
-    const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    const long long t256 = static_cast<long long>(ceil_div(m, kBig)) * ceil_div(n, kBig) * batch;
-    const long long t128 = static_cast<long long>(ceil_div(m, 128)) * ceil_div(n, 128) * batch;
-    return t256 < cus && 4 * t128 >= 3LL * cus && !(s256 > 1 && kc256 >= 1024);
-}
-
-// K per split slice from which a split 64x64-tile product runs on four wave sets.
-constexpr int kKsSliceMin = 1024;
-
-int splitk_plan(int m, int n, int k, int batch, size_t ws_floats, int* kchunk_out, bool unreduced)
-{
-    const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    const long long tiles64 = static_cast<long long>(ceil_div(m, 64)) * ceil_div(n, 64) * batch;
-    const long long big_tiles = static_cast<long long>(ceil_div(m, 128)) * ceil_div(n, 128) * batch;
-    if (big_tiles >= cus || tiles64 >= cus) return 1;
-    const long long mnb = static_cast<long long>(m) * n * batch;
     const long long tiles32 = static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) * batch;
-    const int pass = 64 * kSmallU;
-    if (unreduced && use_small_kernel(m, n, k) && tiles32 < cus && k > pass) {
-        // 16x16 tiles whose consumer sums the slices itself (no reduce
-        // launch): one software pass per slice, slices a multiple of 64 deep
-        long long s = std::min<long long>(ceil_div(k, pass), 64);
-        if (mnb > 0) s = std::min<long long>(s, static_cast<long long>(ws_floats / mnb));
-        if (s < 2) return 1;
-        const int kchunk = ceil_div(ceil_div(k, static_cast<int>(s)), 64) * 64;
-        const int splits = ceil_div(k, kchunk);
-        if (splits < 2) return 1;
-        *kchunk_out = kchunk;
-        return splits;
-    }
-    long long tiles, min_k;
-    int unit;
-    if (use_small_kernel(m, n, k)) {
-        // 32x32 tiles, K shared by four waves: split only long K (each wave
-        // walks K/4 serially; below 1024 the extra reduce launch costs more
-        // than the shorter walk saves)
-        if (k < 1024) return 1;
-        tiles = static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) * batch;
-        unit = 32;
-        min_k = 256;
-        // 16x16 tiles (fewer 32x32 tiles than CUs) take long K unsplit: their
-        // passes are software-pipelined, which beats a split plus its reduce
-        if (tiles < cus) return 1;
-    } else {
-        // 64x64 tiles, 32-deep K tiles walked by one workgroup
-        tiles = tiles64;
-        unit = 32;
-        min_k = 128;
-        // slices of 1024 or more K at one workgroup per CU run on four wave
-        // sets (ks_slices), which beats two single-set workgroups per CU
-        const long long s1 = (cus + tiles - 1) / tiles;
-        if (k / s1 >= kKsSliceMin) {
-            long long s = std::min<long long>(s1, 64);
-            if (mnb > 0) s = std::min<long long>(s, static_cast<long long>(ws_floats / mnb));
-            if (s >= 2) {
-                const int kchunk = ceil_div(ceil_div(k, s), 32) * 32;
-                const int splits = ceil_div(k, kchunk);
-                if (splits >= 2) {
-                    *kchunk_out = kchunk;
-                    return splits;
-                }
-            }
-        }
-    }
-    long long s = (2LL * cus + tiles - 1) / tiles;          // aim at ~2 workgroups per CU
-    s = std::min<long long>(s, k / min_k);
-    s = std::min<long long>(s, 64);
-    if (mnb > 0) s = std::min<long long>(s, static_cast<long long>(ws_floats / mnb));
-    if (s < 2) return 1;
-    const int kchunk = ceil_div(ceil_div(k, s), unit) * unit;
-    const int splits = ceil_div(k, kchunk);
-    if (splits < 2) return 1;
-    *kchunk_out = kchunk;
-    return splits;
+    if (tiles32 >= cus) return false;
+    if (k <= 1024 || (k <= 2048 && vecA && vecB)) return true;
+    return k <= 4096 && !tb && ((ta && vecA && vecB) || (n <= 16 && vecA));
+}
+
+// Up to 16 rows of C the product is one streaming pass over B; from 17 to 32
+// rows that form is level with the three-term kernel on a large aligned B
+// (32x4096x1024 13.0 us against 13.8, 32x4096x4096 27.8 against 26.8) and
+// behind it elsewhere (32x2000x512 12.2 against 10.5, 32x777x1500 15.1 against
+// 11.8), and further behind with more rows (40x4096x4096 32.0 against 27.3).
+bool skinny_best(int m, int n, int k, int vecB)
+{
+    return m <= 16 || (m <= kSkinnyMax && vecB && static_cast<long long>(n) * k >= 1LL << 22);
 }
 
 int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
@@ -2603,16 +1695,17 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
         return fail(LHIP_E_SHAPE, "sgemm: negative batch stride");
     if (o.inner <= 0) return fail(LHIP_E_ARG, "sgemm: inner batch count must be > 0");
     if (o.kblocks <= 0) return fail(LHIP_E_ARG, "sgemm: kblocks must be > 0");
-    const long long big_tiles = static_cast<long long>(ceil_div(m, 128)) * ceil_div(n, 128) * batch;
-    const long long tiles64 = static_cast<long long>(ceil_div(m, 64)) * ceil_div(n, 64) * batch;
-    const int cus = st().cu_count > 0 ? st().cu_count : 256;
     const long long k_all = static_cast<long long>(k) * o.kblocks;
     if (o.kblocks > 1 && k > 0) {
-        // One launch when the small kernel takes the whole K range; otherwise
-        // (transposed A, K not a multiple of 4, or a large problem) the blocks
-        // are accumulated by successive launches.
-        const bool one = !ta && k % 4 == 0 && k_all <= 0x7fffffffLL && big_tiles < cus && tiles64 < cus &&
-                         use_small_kernel(m, n, static_cast<int>(k_all));
+        // One launch where a kernel walks the blocks itself: the three-term
+        // kernel (blocks of whole 16-deep stages), or the 16x16-tile one (A not
+        // transposed, blocks of whole quads).  Otherwise the blocks are
+        // accumulated by successive launches.
+        X3Plan p{};
+        const bool one = k_all <= 0x7fffffffLL &&
+                         (x3_plan(ta, tb, m, n, static_cast<int>(k_all), k, lda, ldb, std::max(ldc, o.ldr), batch, 0, &p) ||
+                          (!ta && k % 4 == 0 &&
+                           tiny_best(ta, tb, m, n, static_cast<int>(k_all), batch, true, true)));
         if (!one) {
             GemmOpts oj = o;
             oj.kblocks = 1;
@@ -2627,6 +1720,7 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
     }
     const bool br = o.kblocks > 1 && k > 0;
     GemmArgs g{};
+
     g.M = m; g.N = n; g.K = static_cast<int>(br ? k_all : k); g.alpha = alpha; g.beta = beta;
     g.Kb = k; g.sAk = br ? o.sAk : 0; g.sBk = br ? o.sBk : 0;
     g.A = A; g.lda = lda; g.sA = sA; g.sA2 = o.sA2;
@@ -2638,70 +1732,44 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
               g.sAk % 4 == 0) ? 1 : 0;
     g.vecB = (k > 0 && ldb % 4 == 0 && aligned16(B) && (batch == 1 || (sB % 4 == 0 && o.sB2 % 4 == 0)) &&
               g.sBk % 4 == 0) ? 1 : 0;
-    // Large problems: 128x128 tiles (64x64 per wave); mid-size: 64x64 tiles;
-    // small (fewer 64x64 tiles than CUs): 32x32 tiles with K shared by the
-    // four waves of a workgroup, split over workgroups when K is very long
-    // (split-K partials in o.ws).
-    if (!br && !o.splits_out && o.ws && ks_split_ok(m, n, k, batch)) {
-        int kc = 0;
-        const int s = ks_split_plan(m, n, k, o.ws_floats, &kc);
-        if (s > 1) {
-            g.splits = s; g.kchunk = kc; g.ws = o.ws;
-            return launch_cfg_ks<64, 64, 32, 4>(ta, tb, g, batch, stream);
-        }
+    if (k == 0) {
+        // C = beta * C through the 16x16-tile kernel
+        if (o.splits_out) *o.splits_out = 1;
+        g.splits = 1;
+        return launch_tiny(ta, tb, g, batch, stream);
     }
-    if (skinny_ok(ta, tb, m, n, batch, br ? o.kblocks : 1) && !o.splits_out && k > 0) {
+    if (!br && !o.splits_out && skinny_ok(ta, tb, m, n, batch, 1) && skinny_best(m, n, k, g.vecB)) {
         g.ws = o.ws;
         g.ws_floats_avail = o.ws ? o.ws_floats : 0;
         return launch_skinny(ta, g, stream);
     }
-    const long long tiles256 = static_cast<long long>(ceil_div(m, kBig)) * ceil_div(n, kBig) * batch;
-    if (tiles256 >= cus) return launch_256(ta, tb, g, batch, stream);
-    int kc256 = 0;
-    const int s256 = (!br && o.ws && !o.splits_out) ? split256_plan(m, n, k, batch, o.ws_floats, &kc256) : 1;
-    if (!br && big128_ok(m, n, batch, s256, kc256)) return launch_big<128>(ta, tb, g, batch, stream);
-    if (s256 > 1) {
-        g.splits = s256; g.kchunk = kc256; g.ws = o.ws;
-        return launch_256(ta, tb, g, batch, stream);
-    }
-    if (!br && o.ws && !o.splits_out && batch == 1) {
-        int kc128 = 0;
-        const int s128 = big128_split_plan(m, n, k, o.ws_floats, &kc128);
-        if (s128 > 1) {
-            g.splits = s128; g.kchunk = kc128; g.ws = o.ws;
-            return launch_big<128>(ta, tb, g, 1, stream);
+    if (o.splits_out && (alpha != 1.f || beta != 0.f || batch != 1 || o.R))
+        return fail(LHIP_E_ARG, "sgemm: unreduced split-K needs alpha 1, beta 0, batch 1");
+    // (the 16x16-tile kernel walks the blocks of a batch-reduce for a plain A only)
+    X3Plan x3{};
+    if ((!(br && (ta || k % 4 != 0)) && tiny_best(ta, tb, m, n, g.K, batch, g.vecA, g.vecB)) ||
+        !x3_plan(ta, tb, m, n, g.K, br ? k : 0, lda, ldb, std::max(ldc, o.ldr), batch,
+                 o.ws ? std::min(o.ws_floats, kX3WsFloats) : 0, &x3)) {
+        g.splits = o.ws && o.splits_out ? tiny_unreduced_plan(m, n, g.K, o.ws_floats, &g.kchunk) : 1;
+        g.ws = o.ws;
+        if (o.splits_out) {
+            *o.splits_out = g.splits > 1 ? g.splits : 1;
+            g.skip_reduce = g.splits > 1 ? 1 : 0;
         }
+        return launch_tiny(ta, tb, g, batch, stream);
     }
-    if (big_tiles >= cus) return launch_cfg<128, 128, 32>(ta, tb, g, batch, stream);
-    // short K (e.g. the LM head, K = dim): the whole K range in one LDS tile,
-    // so a workgroup waits on one load round trip instead of one per 32-deep chunk
-    if (tiles64 >= cus) {
-        // exactly one 64x64 tile per CU: two wave sets per tile, each taking
-        // every other 32-deep chunk (the C2 tied head, 512x2000x128: 1 us less
-        // per step; 1024^3 27.6-27.7 us against 28.9-29.1 on four sets, and
-        // 3-5% at 512x2048x1024 and 2048x512x768); up to two tiles per CU with
-        // long K: two wave sets as well
-        if (g.K >= 64 && tiles64 <= cus) return launch_cfg_ks<64, 64, 32, 2>(ta, tb, g, batch, stream);
-        if (g.K >= 512 && tiles64 <= 2 * cus) return launch_cfg_ks<64, 64, 32, 2>(ta, tb, g, batch, stream);
-        // otherwise one wave set: the same kernel's two-chunk-ahead,
-        // whole-chunk loads (1536^3 104.5 -> 84.7 us, 1600x1600x800 56.7 ->
-        // 47.2 against the single-buffered 64x64 kernel)
-        return launch_cfg_ks<64, 64, 32, 1>(ta, tb, g, batch, stream);
+    if (!br && ks_best(ta, tb, m, n, k, batch, g.vecA, g.vecB)) {
+        if (o.splits_out) *o.splits_out = 1;
+        return launch_ks(ta, tb, g, batch, stream);
     }
-    const bool small = use_small_kernel(m, n, g.K);
-    g.splits = o.ws ? splitk_plan(m, n, g.K, batch, o.ws_floats, &g.kchunk, o.splits_out != nullptr) : 1;
+    g.splits = x3.splits;
+    g.kchunk = x3.kchunk;
     g.ws = o.ws;
     if (o.splits_out) {
-        if (alpha != 1.f || beta != 0.f || batch != 1 || o.R)
-            return fail(LHIP_E_ARG, "sgemm: unreduced split-K needs alpha 1, beta 0, batch 1");
-        *o.splits_out = g.splits > 1 ? g.splits : 1;
-        g.skip_reduce = g.splits > 1 ? 1 : 0;
+        *o.splits_out = x3.splits;
+        g.skip_reduce = x3.splits > 1 ? 1 : 0;
     }
-    const long long tiles32 = static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) * batch;
-    if (small && tiles32 < cus) return launch_tiny(ta, tb, g, batch, stream);
-    if (small) return launch_small(ta, tb, g, batch, stream);
-    if (g.splits > 1 && g.kchunk >= kKsSliceMin) return launch_cfg_ks<64, 64, 32, 4>(ta, tb, g, batch, stream);
-    return launch_cfg_ks<64, 64, 32, 1>(ta, tb, g, batch, stream);
+    return launch_x3(x3.tile, br, ta, tb, g, batch, stream);
 }
 
 int sgemm_launch(int ta, int tb, int m, int n, int k, float alpha,
@@ -2715,7 +1783,7 @@ int sgemm_launch(int ta, int tb, int m, int n, int k, float alpha,
 }
 
 // Fixed split-K scratch of lhip_sgemm_noalloc (the array itself is below, at file scope).
-constexpr size_t kNoallocScratchBytes = static_cast<size_t>(64) << 20;   // 64 MiB
+constexpr size_t kNoallocScratchBytes = kX3WsFloats * sizeof(float);   // 64 MiB
 constexpr int kNoallocMaxDevices = 64;
 
 }  // namespace lhip
@@ -2752,30 +1820,24 @@ int noalloc_scratch_init(int device)
     return LHIP_OK;
 }
 
-// The split-K plan of an immediate product: the slice count (1 = unsplit) and
-// the partials it needs, in floats.  lhip_sgemm and lhip_sgemm_noalloc share
-// it, so both sum the same slices in the same order.
-int immediate_plan(int transa, int transb, int m, int n, int k, int batch, size_t* need_floats)
+size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, size_t head)
 {
-    *need_floats = 0;
-    if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 1;
-    const size_t cap = static_cast<size_t>(1) << 26;
-    int kchunk = 0, splits = 1;
-    if (ks_split_ok(m, n, k, batch)) {
-        splits = ks_split_plan(m, n, k, cap, &kchunk);
-        if (splits <= 1 && skinny_ok(transa, transb, m, n, batch, 1)) splits = skinny_plan(m, n, k, cap, &kchunk);
-    } else if (skinny_ok(transa, transb, m, n, batch, 1)) {
-        splits = skinny_plan(m, n, k, cap, &kchunk);
-    } else {
-        splits = split256_plan(m, n, k, batch, cap, &kchunk);
-        if (big128_ok(m, n, batch, splits, kchunk)) splits = 1;
-        else if (splits <= 1) {
-            splits = batch == 1 ? big128_split_plan(m, n, k, cap, &kchunk) : 1;
-            if (splits <= 1) splits = splitk_plan(m, n, k, batch, cap, &kchunk);
-        }
+    if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 0;
+    const size_t doc = documented_partials(transa, transb, m, n, k, batch);
+    size_t need = 0;
+    X3Plan p{};
+    if (!tiny_best(transa, transb, m, n, k, batch, 0, 0) &&
+        x3_plan(transa, transb, m, n, k, 0, lda, ldb, n, batch, kX3WsFloats, &p) && p.splits > 1)
+        need = static_cast<size_t>(p.splits) * m * n * batch;
+    if (skinny_ok(transa, transb, m, n, batch, 1)) {
+        int kchunk = 0;
+        const int s = skinny_plan(m, n, k, static_cast<size_t>(1) << 26, &kchunk);
+        if (s > 1) need = std::max(need, static_cast<size_t>(s) * m * n);
     }
-    if (splits > 1) *need_floats = static_cast<size_t>(splits) * m * n * batch;
-    return splits;
+    // A recording cannot grow the workspace: products that never needed any
+    // are recorded with what is held (unsplit if need be).
+    if (st().recording && (head + std::max(doc, need)) * sizeof(float) > st().work_bytes) return doc;
+    return std::max(doc, need);
 }
 
 }  // namespace lhip
@@ -2793,9 +1855,8 @@ static int sgemm_immediate(int transa, int transb, int m, int n, int k, float al
 {
     lhip::GemmOpts o;
     o.inner = batch > 0 ? batch : 1;
-    size_t need = 0;
-    if (lhip::immediate_plan(transa, transb, m, n, k, batch, &need) > 1) {
-        o.ws_floats = need;
+    o.ws_floats = lhip::immediate_ws(transa, transb, m, n, k, batch, lda, ldb, 0);
+    if (o.ws_floats > 0) {
         int rc = lhip::workspace(o.ws_floats * sizeof(float), reinterpret_cast<void**>(&o.ws));
         if (rc != LHIP_OK) return rc;
     }
@@ -2811,15 +1872,13 @@ LHIP_API int lhip_sgemm_noalloc(int transa, int transb, int m, int n, int k, flo
     float* const ptr = lhip::g_scratch_dev[st().device];
     if (!ptr) return fail(LHIP_E_DEVICE, "lhip_sgemm_noalloc: scratch of device %d not resolved", st().device);
     lhip::GemmOpts o;
-    size_t need = 0;
-    if (lhip::immediate_plan(transa, transb, m, n, k, 1, &need) > 1) {
-        if (need * sizeof(float) > lhip::kNoallocScratchBytes)
-            return fail(LHIP_E_CAPACITY,
-                        "lhip_sgemm_noalloc: m=%d n=%d k=%d needs %zu bytes of split-K scratch, beyond its fixed "
-                        "%zu bytes; use lhip_sgemm", m, n, k, need * sizeof(float), lhip::kNoallocScratchBytes);
-        o.ws = ptr;
-        o.ws_floats = need;
-    }
+    const size_t need = m > 0 && n > 0 && k > 0 ? lhip::documented_partials(transa, transb, m, n, k, 1) : 0;
+    if (need * sizeof(float) > lhip::kNoallocScratchBytes)
+        return fail(LHIP_E_CAPACITY,
+                    "lhip_sgemm_noalloc: m=%d n=%d k=%d needs %zu bytes of split-K scratch, beyond its fixed "
+                    "%zu bytes; use lhip_sgemm", m, n, k, need * sizeof(float), lhip::kNoallocScratchBytes);
+    o.ws = ptr;
+    o.ws_floats = lhip::kX3WsFloats;
     return lhip::sgemm_run(transa, transb, m, n, k, alpha, A, lda, 0, B, ldb, 0, beta, C, ldc, 0, 1, o,
                            st().stream);
 }

@@ -350,12 +350,9 @@ int sgemm_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream,
 int sgemm_run(int transa, int transb, int m, int n, int k, float alpha,
               const float* A, int lda, long long sA, const float* B, int ldb, long long sB, float beta,
               float* C, int ldc, long long sC, int batch, const GemmOpts& o, hipStream_t stream);
-// The split-K plan of an immediate product (lhip_sgemm's): slice count (1 =
-// unsplit) and, in *need_floats, the partials it needs.
-int immediate_plan(int transa, int transb, int m, int n, int k, int batch, size_t* need_floats);
-// Number of K slices sgemm_run would use (1 = none); *kchunk receives the slice length.
-int splitk_plan(int m, int n, int k, int batch, size_t ws_floats, int* kchunk, bool unreduced = false);
-int split256_plan(int m, int n, int k, int batch, size_t ws_floats, int* kchunk);
+// Floats of split-K workspace an immediate product (lhip_sgemm's) asks for,
+// next to `head` floats the caller needs itself.
+size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, size_t head);
 
 int sgemm_launch(int transa, int transb, int m, int n, int k, float alpha,
                  const float* A, int lda, const float* B, int ldb, float beta,
