@@ -10,6 +10,7 @@
 // leading dimensions, rope :719-767 with pos_ids / pos_offset / half-split /
 // inverse, embed :771-806).
 #include <cmath>
+#include <type_traits>
 
 #include "lhip_internal.h"
 
@@ -452,59 +453,116 @@ __global__ void embed_fwd_kernel(const float* __restrict__ table, const int* __r
 }
 
 // dtable[v] (+)= scale * sum over tokens i with ids[i] == v, added in token
-// order (the Lua loop order, tensor2.lua:592-607), one wave per vocabulary row:
-// the ids are loaded 1024 at a time (16 per lane, all issued before the first
-// compare) and matches found 64 at a time with a wave ballot.  No atomics, so
-// the result is deterministic.  Ids outside [0, vocab) are skipped.
-constexpr int kEmbedChunk = 512;  // columns per pass (8 per lane)
-constexpr int kEmbedIds = 16;     // id chunks of 64 per scan pass
+// order (the Lua loop order, tensor2.lua:592-607).  No atomics, so the result
+// is deterministic.  Ids outside [0, vocab) are skipped.
+//
+// A workgroup owns `rpw` consecutive table rows.  It reads 2048 ids at a time
+// (8 per thread, all issued before the first compare) and lists the tokens of
+// its rows in LDS in token order; then each wave takes (row, 256-column block)
+// pairs, picks the row's tokens out of the list and adds their gradient rows,
+// kEmbedFly of them in flight.  What bounds it: a frequent token's rows are one
+// serial sum, so its loads must overlap; beyond that, the table's one write.
+// 2048 tokens of natural-text skew into 32000x256: 118 us with a wave per row
+// taking one token's row at a time, 22.5 us now (33 MB written: 1.5 TB/s).
+constexpr int kEmbedIds = 8;                     // ids per thread and scan
+constexpr int kEmbedScan = 256 * kEmbedIds;
+constexpr int kEmbedFly = 16;                    // gradient rows in flight per wave
 
-__global__ void __launch_bounds__(64)
-embed_bwd_kernel(const float* __restrict__ g, const int* __restrict__ ids, float* __restrict__ dtable,
-                 int n, int dim, int vocab, float scale, int acc)
+template <bool VEC>
+__global__ void __launch_bounds__(256)
+embed_bwd_kernel(const float* __restrict__ g, const int* __restrict__ ids, float* __restrict__ dtable, int n, int dim,
+                 int vocab, float scale, int acc, int rpw)
 {
-    const int v = blockIdx.x;
-    const int lane = threadIdx.x;
-    for (int d0 = 0; d0 < dim; d0 += kEmbedChunk) {
-        float a[kEmbedChunk / 64];
-        float* row = dtable + static_cast<long long>(v) * dim;
+    __shared__ unsigned list[kEmbedScan];            // row - v0 << 16 | token - c0, in token order
+    __shared__ unsigned short mine[4][kEmbedScan];   // the tokens of a wave's current row
+    __shared__ int count[kEmbedIds * 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1;
+    const int v0 = blockIdx.x * rpw, nrows = min(rpw, vocab - v0);
+    const int blocks = (dim + 255) / 256;
+    for (int c0 = 0; c0 == 0 || c0 < n; c0 += kEmbedScan) {
+        int idv[kEmbedIds];
 #pragma unroll
-        for (int k = 0; k < kEmbedChunk / 64; ++k) {
-            const int d = d0 + lane + 64 * k;
-            a[k] = (acc && d < dim) ? row[d] : 0.f;
+        for (int k = 0; k < kEmbedIds; ++k) {
+            if (c0 + 256 * k >= n) break;            // uniform
+            idv[k] = ids[min(c0 + 256 * k + static_cast<int>(threadIdx.x), n - 1)];
         }
-        for (int c0 = 0; c0 < n; c0 += 64 * kEmbedIds) {
-            int idv[kEmbedIds];
+        unsigned long long hit[kEmbedIds];
 #pragma unroll
-            for (int k = 0; k < kEmbedIds; ++k) {
-                if (c0 + 64 * k >= n) break;                  // uniform
-                const int i = c0 + 64 * k + lane;
-                idv[k] = ids[min(i, n - 1)];
+        for (int k = 0; k < kEmbedIds; ++k) {
+            const int i = c0 + 256 * k + static_cast<int>(threadIdx.x);
+            hit[k] = c0 + 256 * k < n ? __ballot(i < n && idv[k] >= v0 && idv[k] < v0 + nrows) : 0ull;
+            if (lane == 0) count[4 * k + wave] = __popcll(hit[k]);
+        }
+        __syncthreads();
+        // list positions: token order is (k, wave, lane)
+        int total = 0;
+#pragma unroll
+        for (int k = 0; k < kEmbedIds; ++k) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                if (w == wave && (hit[k] >> lane & 1))
+                    list[total + __popcll(hit[k] & below)] =
+                        static_cast<unsigned>(idv[k] - v0) << 16 | static_cast<unsigned>(256 * k + threadIdx.x);
+                total += count[4 * k + w];
             }
+        }
+        __syncthreads();
+        const bool keep = acc || c0 > 0;             // add into the row, or start it from zero
+        for (int p = wave; p < nrows * blocks; p += 4) {
+            const int r = p / blocks, d0 = (p - r * blocks) * 256;
+            int m = 0;
+            for (int i = 0; i < total; i += 64) {
+                const unsigned e = list[min(i + lane, total - 1)];
+                const unsigned long long mk = __ballot(i + lane < total && static_cast<int>(e >> 16) == r);
+                if (mk >> lane & 1) mine[wave][m + __popcll(mk & below)] = static_cast<unsigned short>(e & 0xffffu);
+                m += __popcll(mk);
+            }
+            if (m == 0 && keep) continue;            // the row stays as it is
+            float* row = dtable + static_cast<long long>(v0 + r) * dim;
+            int d[4];
 #pragma unroll
-            for (int k = 0; k < kEmbedIds; ++k) {
-                if (c0 + 64 * k >= n) break;
-                const int i0 = c0 + 64 * k;
-                unsigned long long mask = __ballot(i0 + lane < n && idv[k] == v);
-                while (mask) {
-                    const int b = __ffsll(static_cast<long long>(mask)) - 1;
-                    mask &= mask - 1;
-                    const float* gr = g + static_cast<long long>(i0 + b) * dim;
+            for (int j = 0; j < 4; ++j) d[j] = VEC ? d0 + 4 * lane + j : d0 + lane + 64 * j;
+            const bool in = VEC ? d[0] < dim : true;
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+            if (keep) {
 #pragma unroll
-                    for (int j = 0; j < kEmbedChunk / 64; ++j) {
-                        const int d = d0 + lane + 64 * j;
-                        if (d < dim) a[j] = a[j] + scale * gr[d];
+                for (int j = 0; j < 4; ++j) a[j] = d[j] < dim ? row[d[j]] : 0.f;
+            }
+            // whole batches, then the rest four at a time (the last token's row
+            // again past the end, not added)
+            auto batch = [&](int q, auto nc) {
+                constexpr int N = decltype(nc)::value;
+                float t[N][4];
+#pragma unroll
+                for (int u = 0; u < N; ++u) {
+                    const float* gr = g + static_cast<long long>(c0 + mine[wave][min(q + u, m - 1)]) * dim;
+                    if (VEC) {
+                        const float4 x = *reinterpret_cast<const float4*>(gr + (in ? d[0] : 0));
+                        t[u][0] = x.x; t[u][1] = x.y; t[u][2] = x.z; t[u][3] = x.w;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) t[u][j] = gr[min(d[j], dim - 1)];
                     }
                 }
+#pragma unroll
+                for (int u = 0; u < N; ++u)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) a[j] = q + u < m ? a[j] + scale * t[u][j] : a[j];
+            };
+            int q = 0;
+            for (; q + kEmbedFly <= m; q += kEmbedFly) batch(q, std::integral_constant<int, kEmbedFly>{});
+            for (; q < m; q += 4) batch(q, std::integral_constant<int, 4>{});
+            if (VEC) {
+                if (in) st_stream(row + d[0], make_float4(a[0], a[1], a[2], a[3]));
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (d[j] < dim) row[d[j]] = a[j];
             }
         }
-#pragma unroll
-        for (int k = 0; k < kEmbedChunk / 64; ++k) {
-            const int d = d0 + lane + 64 * k;
-            if (d < dim) row[d] = a[k];
-        }
+        __syncthreads();
     }
-    (void)vocab;
 }
 
 }  // namespace
@@ -636,7 +694,13 @@ int embed_bwd(const float* g, const int* ids, float* dtable, int n, int dim, int
     if (n < 0 || dim <= 0 || vocab <= 0) return fail(LHIP_E_SHAPE, "embed_bwd: n=%d dim=%d vocab=%d", n, dim, vocab);
     if (!dtable) return fail(LHIP_E_NULL, "embed_bwd: dtable is NULL");
     if (n > 0 && (!g || !ids)) return fail(LHIP_E_NULL, "embed_bwd: NULL g/ids");
-    klaunch(embed_bwd_kernel, vocab, 64, 0, s, g, ids, dtable, n, dim, vocab, scale, acc);
+    // one row per wave while the id scans of that many workgroups stay cheap,
+    // sixteen rows per workgroup on large tables
+    const int rpw = vocab <= 8192 ? 4 : 16;
+    if (dim % 4 == 0 && aligned16(g) && aligned16(dtable))
+        klaunch(embed_bwd_kernel<true>, ceil_div(vocab, rpw), 256, 0, s, g, ids, dtable, n, dim, vocab, scale, acc, rpw);
+    else
+        klaunch(embed_bwd_kernel<false>, ceil_div(vocab, rpw), 256, 0, s, g, ids, dtable, n, dim, vocab, scale, acc, rpw);
     return check_launch("embed_bwd");
 }
 
