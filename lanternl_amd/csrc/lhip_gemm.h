@@ -53,6 +53,8 @@ struct X3Plan {
 // offsets, partial stages in a batch-reduce).
 bool x3_plan(int ta, int tb, int m, int n, int k, int kb, int lda, int ldb, int ldc, int batch, size_t ws_floats,
              X3Plan* out);
+// Grouped A^T.B products on it (offsets within the limits of x3_plan's operands).
+int launch_x3_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream);
 int launch_x3(int tile, bool br, int ta, int tb, const GemmArgs& g, int batch, hipStream_t stream);
 
 // K slices of the skinny path (lhip_gemm.hip).

@@ -1558,6 +1558,17 @@ int sgemm_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream,
     // workgroup per CU; 32x32 otherwise
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
     const bool wide = vec && 4 * tiles64 >= cus && tiles64 <= cus;
+    // More than one 64x64 tile per CU, or operands that take no float4 loads:
+    // the three-term kernel (29 products of a 4000x512x4 model over 2048
+    // tokens: 674 us on the 32x32 tiles, 316 us on this)
+    bool x3 = tiles64 > cus || (!vec && 4 * tiles64 >= cus);
+    for (int i = 0; i < ngroups; ++i)
+        x3 = x3 && std::max({g[i].lda, g[i].ldb, 8 * g[i].ldc}) < 1 << 25;
+    if (x3) {
+        if (int rc = launch_x3_grouped_tn(g, ngroups, K, stream)) return rc;
+        if (!cs || cs->njobs <= 0) return LHIP_OK;
+        return rmsnorm_bwd_colsum_multi(cs->partial, cs->nparts, cs->out, cs->njobs, cs->cols, cs->acc, stream);
+    }
     const int tile = wide ? 64 : kGroupedTile;
     long long tiles = 0;
     for (int i = 0; i < ngroups; ++i) {

@@ -175,8 +175,7 @@ struct X3Stage {
 // stages s, s + KS, ... in LDS buffers of its own, the sets' tiles added in set
 // order at the end.
 template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR, bool TA, bool TB>
-__global__ void __launch_bounds__(64 * WM * WN * KS)
-sgemm_x3_kernel(const GemmArgs g, const unsigned kb_magic)
+__device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_magic, const int tm, const int tn)
 {
     constexpr int NT = 64 * WM * WN;
     constexpr int FM = BM / WM / 32, FN = BN / WN / 32;
@@ -194,8 +193,6 @@ sgemm_x3_kernel(const GemmArgs g, const unsigned kb_magic)
     const int lr = lane & 31, h = lane >> 5;
     char* lds = lds_all + set * SET;
 
-    int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
     const long long zo = blockIdx.y / g.inner, zi = blockIdx.y % g.inner;
@@ -487,6 +484,45 @@ sgemm_x3_kernel(const GemmArgs g, const unsigned kb_magic)
     }
 }
 
+template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR, bool TA, bool TB>
+__global__ void __launch_bounds__(64 * WM * WN * KS)
+sgemm_x3_kernel(const GemmArgs g, const unsigned kb_magic)
+{
+    int tm, tn;
+    tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
+    x3_tile<BM, BN, WM, WN, KS, PF, BR, TA, TB>(g, kb_magic, tm, tn);
+}
+
+// Grouped C_g = A_g^T . B_g over the same K (the weight gradients of a training
+// step in one launch): workgroup id -> (group, tile) through the groups'
+// first-tile table, XCD-contiguous so that an XCD works on neighbouring tiles.
+struct X3GroupArgs {
+    const float* A[kGroupedMax];
+    const float* B[kGroupedMax];
+    float* C[kGroupedMax];
+    int lda[kGroupedMax], ldb[kGroupedMax], ldc[kGroupedMax], M[kGroupedMax], N[kGroupedMax];
+    int tile0[kGroupedMax + 1], tiles_m[kGroupedMax];
+    int ngroups, K;
+};
+
+template <int BT, int WM, int WN, int KS>
+__global__ void __launch_bounds__(64 * WM * WN * KS)
+sgemm_x3_grouped_kernel(const X3GroupArgs ga)
+{
+    const int pid = static_cast<int>(blockIdx.x % 8) * static_cast<int>(gridDim.x / 8) + static_cast<int>(blockIdx.x / 8);
+    if (pid >= ga.tile0[ga.ngroups]) return;
+    int e = 0;
+    while (pid >= ga.tile0[e + 1]) ++e;
+    GemmArgs g{};
+    g.M = ga.M[e]; g.N = ga.N[e]; g.K = ga.K; g.Kb = ga.K; g.alpha = 1.f;
+    g.A = ga.A[e]; g.lda = ga.lda[e];
+    g.B = ga.B[e]; g.ldb = ga.ldb[e];
+    g.C = ga.C[e]; g.ldc = ga.ldc[e];
+    g.inner = 1; g.splits = 1; g.kchunk = ga.K;
+    const int t = pid - ga.tile0[e];
+    x3_tile<BT, BT, WM, WN, KS, 2, false, true, false>(g, 0, t % ga.tiles_m[e], t / ga.tiles_m[e]);
+}
+
 template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR = false>
 int launch_cfg_x3(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
 {
@@ -579,6 +615,38 @@ int launch_x3(int tile, bool br, int ta, int tb, const GemmArgs& g, int batch, h
         }
     };
     return br ? go(std::true_type{}) : go(std::false_type{});
+}
+
+// 128x128 tiles once they fill the CUs (each then costs 0.62 us per stage and
+// workgroup), 64x64 tiles on two wave sets below that.
+int launch_x3_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream)
+{
+    const int cus = st().cu_count > 0 ? st().cu_count : 256;
+    auto count = [&](int tile) {
+        long long n = 0;
+        for (int i = 0; i < ngroups; ++i) n += static_cast<long long>(ceil_div(g[i].M, tile)) * ceil_div(g[i].N, tile);
+        return n;
+    };
+    const int tile = 4 * count(128) >= 3LL * cus ? 128 : 64;
+    const long long tiles = count(tile);
+    if (tiles > 0x7ffffff0LL) return fail(LHIP_E_CAPACITY, "sgemm_grouped_tn: too many tiles");
+    X3GroupArgs ga{};
+    int first = 0;
+    for (int i = 0; i < ngroups; ++i) {
+        ga.A[i] = g[i].A; ga.B[i] = g[i].B; ga.C[i] = g[i].C;
+        ga.lda[i] = g[i].lda; ga.ldb[i] = g[i].ldb; ga.ldc[i] = g[i].ldc;
+        ga.M[i] = g[i].M; ga.N[i] = g[i].N;
+        ga.tile0[i] = first;
+        ga.tiles_m[i] = ceil_div(g[i].M, tile);
+        first += ga.tiles_m[i] * ceil_div(g[i].N, tile);
+    }
+    ga.tile0[ngroups] = first;
+    ga.ngroups = ngroups;
+    ga.K = K;
+    const unsigned grid = (static_cast<unsigned>(first) + 7u) / 8u * 8u;
+    if (tile == 128) klaunch(sgemm_x3_grouped_kernel<128, 2, 4, 1>, grid, 512, 0, stream, ga);
+    else klaunch(sgemm_x3_grouped_kernel<64, 2, 2, 2>, grid, 512, 0, stream, ga);
+    return check_launch("sgemm_grouped_tn (x3)");
 }
 
 }  // namespace lhip

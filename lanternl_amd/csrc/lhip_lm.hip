@@ -692,7 +692,15 @@ LHIP_API int lhip_lm_create(const lhip_lm_config_t* cfg, void** model)
         }
     }
     m->fused_attn = lhip::attn_fused_ok(m->T, m->hd);
-    m->fused_gemm = lhip::lm_fuse_ok(m->D, m->D, m->D) && m->F % 4 == 0;
+    // The fused 16x16-tile GEMMs save a launch per norm, gate and norm
+    // backward; with enough rows the separate kernels and the larger tiles are
+    // faster (step, us, fused and separate): dim 128 with 1024 rows 331 and
+    // 389, 2048 rows 589 and 594; dim 256 with 512 rows 482 and 526, 1024 rows
+    // 761 and 673; dim 512 with 256 rows 439 and 445, 512 rows 604 and 489,
+    // 2048 rows 3246 and 1874; dim 64 with 4096 rows 307 and 331.
+    const long long rows = static_cast<long long>(m->N) * m->D;
+    m->fused_gemm = lhip::lm_fuse_ok(m->D, m->D, m->D) && m->F % 4 == 0 &&
+                    !((m->D >= 256 && rows >= 1LL << 18) || (m->D >= 128 && rows >= 1LL << 19));
     m->h_tgt.assign(static_cast<size_t>(N), 0);
     m->h_len.assign(static_cast<size_t>(m->B), 0);
     *model = m;
