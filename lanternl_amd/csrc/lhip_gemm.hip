@@ -1657,9 +1657,12 @@ int tiny_unreduced_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
     return ceil_div(k, kchunk);
 }
 
-// Products with fewer 32x32 tiles than CUs that stay on 16x16 tiles: four
-// times the workgroups, and up to K = 512 one round trip of loads.  K up to
-// 1024; up to 2048 when both operands take float4 loads (256x256x1536 NT 11.1
+// Products with few 32x32 tiles that stay on 16x16 tiles: four times the
+// workgroups, and up to K = 512 one round trip of loads.  Up to two tiles per CU
+// with K up to 256, or 512 for the first quarter past one (512x640x256 NN 6.0 us
+// against 8.5, 512x512x512 8.5 against 12.1, 521x665x186 TN 6.8 against 9.3, but
+// unaligned NT 8.9 against 7.2; 800x800x130, 2.4 tiles per CU, 8.9 against 7.5).
+// With fewer tiles than CUs K up to 1024; up to 2048 when both operands take float4 loads (256x256x1536 NT 11.1
 // us against 12.1 on the three-term kernel, 512x128x2000 10.2 against 11.6;
 // unaligned 238x474x1199 28.4 against 12.4); up to 4096 where B is read along
 // its rows and the product is one column tile wide, or A is K-major
@@ -1669,7 +1672,8 @@ bool tiny_best(int ta, int tb, int m, int n, int k, int batch, int vecA, int vec
 {
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
     const long long tiles32 = static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) * batch;
-    if (tiles32 >= cus) return false;
+    if (tiles32 >= cus)
+        return tiles32 < 2 * cus && ((k <= 256 && (!tb || (vecA && vecB))) || (!tb && k <= 512 && 4 * tiles32 <= 5 * cus));
     if (k <= 1024 || (k <= 2048 && vecA && vecB)) return true;
     return k <= 4096 && !tb && ((ta && vecA && vecB) || (n <= 16 && vecA));
 }
@@ -1758,7 +1762,12 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
         return fail(LHIP_E_ARG, "sgemm: unreduced split-K needs alpha 1, beta 0, batch 1");
     // (the 16x16-tile kernel walks the blocks of a batch-reduce for a plain A only)
     X3Plan x3{};
-    if ((!(br && (ta || k % 4 != 0)) && tiny_best(ta, tb, m, n, g.K, batch, g.vecA, g.vecB)) ||
+    // An unreduced split of a small product: one-pass slices on 16x16 tiles, at
+    // any K they cover.
+    const int cus = st().cu_count > 0 ? st().cu_count : 256;
+    const bool tiny_slices = o.splits_out && o.ws && k <= 64 * 64 * kSmallU &&
+                             static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) < cus && (m <= 64 || n <= 64);
+    if (tiny_slices || (!(br && (ta || k % 4 != 0)) && tiny_best(ta, tb, m, n, g.K, batch, g.vecA, g.vecB)) ||
         !x3_plan(ta, tb, m, n, g.K, br ? k : 0, lda, ldb, std::max(ldc, o.ldr), batch,
                  o.ws ? std::min(o.ws_floats, kX3WsFloats) : 0, &x3)) {
         g.splits = o.ws && o.splits_out ? tiny_unreduced_plan(m, n, g.K, o.ws_floats, &g.kchunk) : 1;
