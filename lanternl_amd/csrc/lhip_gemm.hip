@@ -1555,9 +1555,12 @@ int sgemm_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream,
         tiles64 += static_cast<long long>(ceil_div(e.M, 64)) * ceil_div(e.N, 64);
     }
     // 64x64 tiles once they give a quarter of the CUs work and fit one
-    // workgroup per CU; 32x32 otherwise
+    // workgroup per CU, or where K is so short that running the scatter and the
+    // squared norm in the same launch is worth more than the finer tiles
+    // (256x64x2 step, 128 rows: 106 -> 100 us; but 500x64x2, 2048 rows: 178 on
+    // 32x32, 211 on these); 32x32 otherwise
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
-    const bool wide = vec && 4 * tiles64 >= cus && tiles64 <= cus;
+    const bool wide = vec && tiles64 <= cus && (4 * tiles64 >= cus || K <= 256);
     // More than one 64x64 tile per CU, or operands that take no float4 loads:
     // the three-term kernel (29 products of a 4000x512x4 model over 2048
     // tokens: 674 us on the 32x32 tiles, 316 us on this)
