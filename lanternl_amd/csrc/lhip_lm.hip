@@ -60,13 +60,15 @@ __global__ void set_hyper_kernel(float* hp, const Hyper h)
 
 // A batch from its pinned staging slot: ids, targets (n each) and window lengths
 // (b).  The stream runs in order, so when this copy starts every earlier one has
-// finished: block 0 reports that to the host, which may then reuse their slots.
+// finished: block 0 reports that to the host, which may then reuse their slots
+// (a relaxed store: nothing of this kernel's is published by it, and a release
+// would write back the L2s).
 __global__ void __launch_bounds__(256) batch_in_kernel(const int* __restrict__ slot, int* __restrict__ ids,
                                                        int* __restrict__ tgt, int* __restrict__ wlen, int n, int b,
                                                        unsigned* done, unsigned earlier)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i == 0) __hip_atomic_store(done, earlier, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (i == 0) __hip_atomic_store(done, earlier, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (i < n) {
         const int id = slot[i], t = slot[n + i];
         ids[i] = id;
