@@ -36,6 +36,7 @@ struct GemmArgs {
     float* ws;                        // split-K partials [split][batch][M][N]
     int Kb;                           // batch-reduce: K = kblocks * Kb, block j reads A + j*sAk, B + j*sBk
     long long sAk, sBk;
+    int tail;                         // x3: only the last `tail` tiles are split (partials in ws as [slice][tile][tile elements])
     int skip_reduce;                  // split-K slices stay in ws for the caller to sum
     size_t ws_floats_avail;           // floats available at ws (skinny path's split plan)
 };
@@ -47,12 +48,15 @@ constexpr size_t kX3WsFloats = static_cast<size_t>(1) << 24;   // most split-K p
 struct X3Plan {
     int tile;             // index into the kernel's tile table
     int splits, kchunk;   // split-K slices and their length
+    int tail;             // > 0: only the last `tail` tiles are split (the rest run whole)
+    size_t ws_floats;     // the slices' partials
 };
-// kb: the block length of a batch-reduce (0: one block, which may be split).
+// kb: the block length of a batch-reduce (0: one block, which may be split);
+// tail_ok: the last tiles alone may be split (the launch then reduces them itself).
 // False when no tile takes the operands (leading dimensions past 32-bit
 // offsets, partial stages in a batch-reduce).
 bool x3_plan(int ta, int tb, int m, int n, int k, int kb, int lda, int ldb, int ldc, int batch, size_t ws_floats,
-             X3Plan* out);
+             bool tail_ok, X3Plan* out);
 // Grouped A^T.B products on it (offsets within the limits of x3_plan's operands).
 int launch_x3_grouped_tn(const GroupedTN* g, int ngroups, int K, hipStream_t stream);
 int launch_x3(int tile, bool br, int ta, int tb, const GemmArgs& g, int batch, hipStream_t stream);

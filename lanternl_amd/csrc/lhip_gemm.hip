@@ -1721,7 +1721,7 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
         // accumulated by successive launches.
         X3Plan p{};
         const bool one = k_all <= 0x7fffffffLL &&
-                         (x3_plan(ta, tb, m, n, static_cast<int>(k_all), k, lda, ldb, std::max(ldc, o.ldr), batch, 0, &p) ||
+                         (x3_plan(ta, tb, m, n, static_cast<int>(k_all), k, lda, ldb, std::max(ldc, o.ldr), batch, 0, false, &p) ||
                           (!ta && k % 4 == 0 &&
                            tiny_best(ta, tb, m, n, static_cast<int>(k_all), batch, true, true)));
         if (!one) {
@@ -1771,8 +1771,8 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
     const bool tiny_slices = o.splits_out && o.ws && k <= 64 * 64 * kSmallU &&
                              static_cast<long long>(ceil_div(m, 32)) * ceil_div(n, 32) < cus && (m <= 64 || n <= 64);
     if (tiny_slices || (!(br && (ta || k % 4 != 0)) && tiny_best(ta, tb, m, n, g.K, batch, g.vecA, g.vecB)) ||
-        !x3_plan(ta, tb, m, n, g.K, br ? k : 0, lda, ldb, std::max(ldc, o.ldr), batch,
-                 o.ws ? std::min(o.ws_floats, kX3WsFloats) : 0, &x3)) {
+        !(o.plan ? (x3 = *o.plan, true) : x3_plan(ta, tb, m, n, g.K, br ? k : 0, lda, ldb, std::max(ldc, o.ldr), batch,
+                 o.ws ? std::min(o.ws_floats, kX3WsFloats) : 0, !o.splits_out, &x3))) {
         g.splits = o.ws && o.splits_out ? tiny_unreduced_plan(m, n, g.K, o.ws_floats, &g.kchunk) : 1;
         g.ws = o.ws;
         if (o.splits_out) {
@@ -1787,6 +1787,7 @@ int sgemm_run(int ta, int tb, int m, int n, int k, float alpha,
     }
     g.splits = x3.splits;
     g.kchunk = x3.kchunk;
+    g.tail = x3.tail;
     g.ws = o.ws;
     if (o.splits_out) {
         *o.splits_out = x3.splits;
@@ -1843,23 +1844,32 @@ int noalloc_scratch_init(int device)
     return LHIP_OK;
 }
 
-size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, size_t head)
+size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, int ldc, size_t head,
+                    X3Plan* plan, bool* planned)
 {
+    if (planned) *planned = false;
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 0;
     const size_t doc = documented_partials(transa, transb, m, n, k, batch);
     size_t need = 0;
     X3Plan p{};
-    if (!tiny_best(transa, transb, m, n, k, batch, 0, 0) &&
-        x3_plan(transa, transb, m, n, k, 0, lda, ldb, n, batch, kX3WsFloats, &p) && p.splits > 1)
-        need = static_cast<size_t>(p.splits) * m * n * batch;
-    if (skinny_ok(transa, transb, m, n, batch, 1)) {
+    const bool skinny = skinny_ok(transa, transb, m, n, batch, 1);
+    if (skinny) {
         int kchunk = 0;
         const int s = skinny_plan(m, n, k, static_cast<size_t>(1) << 26, &kchunk);
-        if (s > 1) need = std::max(need, static_cast<size_t>(s) * m * n);
+        if (s > 1) need = static_cast<size_t>(s) * m * n;
+    }
+    bool ok = false;
+    if (!(skinny && m <= 16) && !tiny_best(transa, transb, m, n, k, batch, 0, 0)) {
+        ok = x3_plan(transa, transb, m, n, k, 0, lda, ldb, ldc, batch, kX3WsFloats, true, &p);
+        if (ok) need = std::max(need, p.ws_floats);
     }
     // A recording cannot grow the workspace: products that never needed any
     // are recorded with what is held (unsplit if need be).
     if (st().recording && (head + std::max(doc, need)) * sizeof(float) > st().work_bytes) return doc;
+    if (ok && plan) {
+        *plan = p;
+        *planned = true;
+    }
     return std::max(doc, need);
 }
 
@@ -1878,7 +1888,10 @@ static int sgemm_immediate(int transa, int transb, int m, int n, int k, float al
 {
     lhip::GemmOpts o;
     o.inner = batch > 0 ? batch : 1;
-    o.ws_floats = lhip::immediate_ws(transa, transb, m, n, k, batch, lda, ldb, 0);
+    lhip::X3Plan plan;
+    bool planned = false;
+    o.ws_floats = lhip::immediate_ws(transa, transb, m, n, k, batch, lda, ldb, ldc, 0, &plan, &planned);
+    if (planned) o.plan = &plan;
     if (o.ws_floats > 0) {
         int rc = lhip::workspace(o.ws_floats * sizeof(float), reinterpret_cast<void**>(&o.ws));
         if (rc != LHIP_OK) return rc;

@@ -175,7 +175,8 @@ struct X3Stage {
 // stages s, s + KS, ... in LDS buffers of its own, the sets' tiles added in set
 // order at the end.
 template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR, bool TA, bool TB>
-__device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_magic, const int tm, const int tn)
+__device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_magic, const int tm, const int tn,
+                                        const int kbeg, const int kend, float* const part)
 {
     constexpr int NT = 64 * WM * WN;
     constexpr int FM = BM / WM / 32, FN = BN / WN / 32;
@@ -196,8 +197,7 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_mag
     const int m0 = tm * BM, n0 = tn * BN;
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
     const long long zo = blockIdx.y / g.inner, zi = blockIdx.y % g.inner;
-    const int kbeg = blockIdx.z * g.kchunk;
-    const int K = min(g.K, kbeg + g.kchunk) - kbeg;
+    const int K = kend - kbeg;
     const float* __restrict__ A = g.A + zo * g.sA2 + zi * g.sA + (TA ? m0 : static_cast<long long>(m0) * g.lda) +
                                   (TA ? static_cast<long long>(kbeg) * g.lda : kbeg);
     const float* __restrict__ B = g.B + zo * g.sB2 + zi * g.sB + (TB ? static_cast<long long>(n0) * g.ldb : n0) +
@@ -274,10 +274,10 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_mag
     // set reloads that stage into the idle buffer: no branch holds a load.
     const int nst = K / kX3K;            // whole stages of the slice
     const int tail = K - nst * kX3K;
-    const int iters = (nst + KS - 1) / KS;
+    const int rounds = nst / KS;         // every set has a stage: no branch in the loop
     const int last = nst - 1;
     constexpr int U = SA::U + SB::U;
-    if (iters > 0) {
+    if (nst > 0) {
         // the stage the next load_all takes, and where its operands start
         int c = min(set, last);
         const float* pa = uniform(a_base(c));
@@ -314,28 +314,34 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_mag
             char* nxt = lds + ((t & 1) ^ 1) * BUF;
             Frags cu;
             read_frags(cu, lds + (t & 1) * BUF);
-            // a set past its last stage holds that stage again: leave its sums alone
-            if (KS == 1 || t * KS + set <= last) {
-                mma(cu, 2, 0);
-                if (0 < U) put(f, 0, nxt);
-                mma(cu, 1, 1);
-                if (1 < U) put(f, 1, nxt);
-                mma(cu, 0, 2);
-                if (2 < U) put(f, 2, nxt);
-                mma(cu, 1, 0);
-                if (3 < U) put(f, 3, nxt);
-                load_all(f);
-                mma(cu, 0, 1);
-                mma(cu, 0, 0);
-            }
+            mma(cu, 2, 0);
+            if (0 < U) put(f, 0, nxt);
+            mma(cu, 1, 1);
+            if (1 < U) put(f, 1, nxt);
+            mma(cu, 0, 2);
+            if (2 < U) put(f, 2, nxt);
+            mma(cu, 1, 0);
+            if (3 < U) put(f, 3, nxt);
+            load_all(f);
+            mma(cu, 0, 1);
+            mma(cu, 0, 0);
             __syncthreads();
         };
+        int t = 0;
         if (PF == 1) {
-            for (int t = 0; t < iters; ++t) body(t, 0);
+            for (; t < rounds; ++t) body(t, 0);
         } else {
-            int t = 0;
-            for (; t + 1 < iters; t += 2) { body(t, 1); body(t + 1, 0); }
-            if (t < iters) body(t, 1);
+            for (; t + 1 < rounds; t += 2) { body(t, 1); body(t + 1, 0); }
+            if (t < rounds) body(t++, 1);
+        }
+        // the uneven round of the wave sets: the stage is in LDS already
+        if (KS > 1 && rounds * KS < nst) {
+            if (rounds * KS + set <= last) {
+                Frags cu;
+                read_frags(cu, lds + (rounds & 1) * BUF);
+                mma(cu, 2, 0); mma(cu, 1, 1); mma(cu, 0, 2); mma(cu, 1, 0); mma(cu, 0, 1); mma(cu, 0, 0);
+            }
+            __syncthreads();
         }
     }
     if (tail) {
@@ -446,13 +452,15 @@ __device__ __forceinline__ void x3_tile(const GemmArgs& g, const unsigned kb_mag
     auto store = [&](const __amdgpu_buffer_rsrc_t& rs, float v, int off) {
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, off, 0, 0);
     };
-    // a slice's raw sums go to [slice][batch][M][N]; the ordered reduce applies alpha, beta and R
-    const bool slice = g.splits > 1;
-    const int ld = slice ? g.N : g.ldc;
+    // a slice's raw sums go to its partials ([slice][batch][M][N], or a whole
+    // tile when only the last tiles are split); the ordered reduce applies
+    // alpha, beta and R
+    const bool slice = part != nullptr, whole = slice && g.tail > 0;
+    const int ld = whole ? BN : slice ? g.N : g.ldc;
     const float alpha = slice ? 1.f : g.alpha;
-    const __amdgpu_buffer_rsrc_t rd = tile_rsrc(
-        slice ? g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * (static_cast<long long>(g.M) * g.N)
-              : g.C + coff, ld);
+    const __amdgpu_buffer_rsrc_t rd =
+        whole ? __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(uniform(part)), 0, 4 * BM * BN, 0x00020000)
+              : tile_rsrc(slice ? part : g.C + coff, ld);
     if (slice || g.beta == 0.f) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
@@ -488,9 +496,67 @@ template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR, bool TA, bool
 __global__ void __launch_bounds__(64 * WM * WN * KS)
 sgemm_x3_kernel(const GemmArgs g, const unsigned kb_magic)
 {
+    // One call of the tile below, so that its code is there once.  With a tail
+    // the whole tiles come first (one round of workgroups or more), then the
+    // slices of the rest, which share the CUs with them.
+    int pid = blockIdx.x, npid = gridDim.x, kbeg = blockIdx.z * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+    float* part = nullptr;
+    if (g.tail > 0) {
+        const int whole = g.tiles_m * g.tiles_n - g.tail, e = pid - whole;
+        if (e < 0) {
+            npid = whole;
+            kend = g.K;
+        } else {
+            const int s = e / g.tail, t = e - s * g.tail;
+            pid = whole + t;
+            npid = 1;
+            kbeg = s * g.kchunk;
+            kend = min(g.K, kbeg + g.kchunk);
+            part = g.ws + static_cast<size_t>(e) * (BM * BN);
+        }
+    } else if (g.splits > 1) {
+        part = g.ws + (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * (static_cast<long long>(g.M) * g.N);
+    }
     int tm, tn;
-    tile_coords(blockIdx.x, gridDim.x, g.tiles_m, g.tiles_n, tm, tn);
-    x3_tile<BM, BN, WM, WN, KS, PF, BR, TA, TB>(g, kb_magic, tm, tn);
+    tile_coords(pid, npid, g.tiles_m, g.tiles_n, tm, tn);
+    x3_tile<BM, BN, WM, WN, KS, PF, BR, TA, TB>(g, kb_magic, tm, tn, kbeg, kend, part);
+}
+
+// The ordered sum of the split tiles: C = alpha * sum_s part[s] + beta * R, four
+// columns per thread (tiles are whole rows of float4; C and R take dword-aligned
+// ones), eight slices in flight.
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int BT>
+__global__ void __launch_bounds__(256) x3_tail_reduce(const GemmArgs g)
+{
+    constexpr int PER = BT * BT / 4;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int t = i / PER, q = i - t * PER;
+    int tm, tn;
+    tile_coords(g.tiles_m * g.tiles_n - g.tail + t, 1, g.tiles_m, g.tiles_n, tm, tn);
+    const int row = tm * BT + q / (BT / 4), col = tn * BT + 4 * (q % (BT / 4));
+    if (row >= g.M || col >= g.N) return;
+    const floatx4* src = reinterpret_cast<const floatx4*>(g.ws) + static_cast<size_t>(t) * PER + q;
+    const size_t step = static_cast<size_t>(g.tail) * PER;
+    floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < g.splits; s += 8) {
+        floatx4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = src[min(s + u, g.splits - 1) * step];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + u < g.splits) sum += v[u];
+    }
+    float* dst = g.C + static_cast<long long>(row) * g.ldc + col;
+    const float* r = g.R ? g.R + static_cast<long long>(row) * g.ldr + col : dst;
+    if (col + 4 <= g.N) {
+        floatx4 o = g.alpha * sum;
+        if (g.beta != 0.f) o += g.beta * static_cast<floatx4>(*reinterpret_cast<const floatx4u*>(r));
+        *reinterpret_cast<floatx4u*>(dst) = o;
+    } else {
+        for (int c = 0; col + c < g.N; ++c) dst[c] = g.beta != 0.f ? g.alpha * sum[c] + g.beta * r[c] : g.alpha * sum[c];
+    }
 }
 
 // Grouped C_g = A_g^T . B_g over the same K (the weight gradients of a training
@@ -520,7 +586,7 @@ sgemm_x3_grouped_kernel(const X3GroupArgs ga)
     g.C = ga.C[e]; g.ldc = ga.ldc[e];
     g.inner = 1; g.splits = 1; g.kchunk = ga.K;
     const int t = pid - ga.tile0[e];
-    x3_tile<BT, BT, WM, WN, KS, 2, false, true, false>(g, 0, t % ga.tiles_m[e], t / ga.tiles_m[e]);
+    x3_tile<BT, BT, WM, WN, KS, 2, false, true, false>(g, 0, t % ga.tiles_m[e], t / ga.tiles_m[e], 0, ga.K, nullptr);
 }
 
 template <int BM, int BN, int WM, int WN, int KS, int PF, bool BR = false>
@@ -533,12 +599,18 @@ int launch_cfg_x3(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
     if (g.splits <= 1) { g.splits = 1; g.kchunk = g.K; g.ws = nullptr; }
     const int cpb = g.Kb / kX3K;
     const unsigned magic = g.Kb == g.K ? 0u : static_cast<unsigned>(((1ull << 32) + cpb - 1) / cpb);
-    const dim3 grid(static_cast<unsigned>(nwg), batch, g.splits), block(64 * WM * WN * KS, 1, 1);
+    const dim3 grid = g.tail > 0 ? dim3(static_cast<unsigned>(nwg - g.tail + static_cast<long long>(g.tail) * g.splits), 1, 1)
+                                 : dim3(static_cast<unsigned>(nwg), batch, g.splits);
+    const dim3 block(64 * WM * WN * KS, 1, 1);
     if (!ta && !tb) klaunch(sgemm_x3_kernel<BM, BN, WM, WN, KS, PF, BR, false, false>, grid, block, 0, stream, g, magic);
     else if (ta && !tb) klaunch(sgemm_x3_kernel<BM, BN, WM, WN, KS, PF, BR, true, false>, grid, block, 0, stream, g, magic);
     else if (!ta && tb) klaunch(sgemm_x3_kernel<BM, BN, WM, WN, KS, PF, BR, false, true>, grid, block, 0, stream, g, magic);
     else klaunch(sgemm_x3_kernel<BM, BN, WM, WN, KS, PF, BR, true, true>, grid, block, 0, stream, g, magic);
     const int rc = check_launch("sgemm (x3): kernel launch");
+    if (rc == LHIP_OK && g.tail > 0) {
+        klaunch(x3_tail_reduce<BM>, g.tail * (BM * BN / 4 / 256), 256, 0, stream, g);
+        return check_launch("sgemm (x3): reduce");
+    }
     if (rc != LHIP_OK || g.splits <= 1 || g.skip_reduce) return rc;
     return launch_reduce(g, batch, stream);
 }
@@ -567,12 +639,13 @@ constexpr X3Tile kX3Tiles[] = {
 // its traffic.  Against the best of all tiles and splits the choice lost 2% on
 // average over the 68 products, at most 19%.
 bool x3_plan(int ta, int tb, int m, int n, int k, int kb, int lda, int ldb, int ldc, int batch, size_t ws_floats,
-             X3Plan* out)
+             bool tail_ok, X3Plan* out)
 {
     if (kb % kX3K != 0) return false;
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
     const double mnb = static_cast<double>(m) * n * batch;
     static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64, 96, 128};
+    const double per_cus = 1.0 / cus;
     double best = 0.0;
     bool found = false;
     for (int t = 0; t < static_cast<int>(sizeof(kX3Tiles) / sizeof(kX3Tiles[0])); ++t) {
@@ -585,21 +658,48 @@ bool x3_plan(int ta, int tb, int m, int n, int k, int kb, int lda, int ldb, int 
         const double tiles = static_cast<double>(ceil_div(m, c.rows)) * ceil_div(n, c.rows) * batch;
         for (int s : kSplits) {
             if (s > 1 && (kb > 0 || k < 64 * s || s * mnb > static_cast<double>(ws_floats))) break;
-            const int kchunk = ceil_div(ceil_div(k, s), kX3K) * kX3K;
-            const int splits = ceil_div(k, kchunk);
-            const double per_cu = tiles * splits / cus, full = per_cu <= 4.0 ? std::ceil(per_cu) : per_cu + 0.5;
-            if (full > 1.0 && c.shared == 0.0) break;
-            const double stages = kchunk / kX3K;
+            const double per_cu = tiles * s * per_cus, full = per_cu <= 4.0 ? std::ceil(per_cu) : per_cu + 0.5;
+            if (full > 1.0 && (c.shared == 0.0 || s * mnb > 64e6)) break;
+            const int stages = static_cast<int>((static_cast<unsigned>(k) + 16u * s - 1u) / (16u * s));
             double us = c.fixed + stages * (full <= 1.0 ? c.alone : c.shared * full);
-            if (splits > 1) us += 4.0 + (splits + 1) * mnb * 4e-6 / 3.5;   // reduce at 3.5 TB/s
+            if (s > 1) us += 4.0 + (s + 1) * mnb * (4e-6 / 3.5);   // reduce at 3.5 TB/s
             if (!found || us < best) {
                 found = true;
                 best = us;
-                *out = {t, splits, splits > 1 ? kchunk : k};
+                *out = {t, s, stages * kX3K, 0, 0};
             }
         }
+        // Tiles a little past a whole round of CUs: the rounds run whole, the
+        // rest is split so that it fills the CUs once more for a fraction of a
+        // tile's time.
+        const long long rest = static_cast<long long>(tiles) % cus, rounds = static_cast<long long>(tiles) / cus;
+        if (!tail_ok || batch != 1 || kb > 0 || c.shared == 0.0 || rounds < 1 || rounds > 8 || rest == 0) continue;
+        const int s = static_cast<int>(std::min<long long>({cus / rest, k / 64, 32LL}));
+        if (s < 2) continue;
+        const int stages = ceil_div(k, kX3K * s);
+        const double part = static_cast<double>(s) * rest * c.rows * c.rows;
+        if (part > static_cast<double>(ws_floats)) continue;
+        const double us = c.fixed + k / kX3K * (rounds == 1 ? c.alone : c.shared * rounds) + stages * c.shared + 5.0 +
+                          part * (8e-6 / 3.5);
+        if (!found || us < best) {
+            found = true;
+            best = us;
+            *out = {t, s, stages * kX3K, static_cast<int>(rest), 0};
+        }
     }
-    return found;
+    if (!found) return false;
+    // slices are whole stages, so there may be fewer than asked for
+    if (out->splits > 1) out->splits = ceil_div(k, out->kchunk);
+    if (out->splits > 1) {
+        const int rows = kX3Tiles[out->tile].rows;
+        out->ws_floats = out->tail > 0 ? static_cast<size_t>(out->splits) * out->tail * rows * rows
+                                       : static_cast<size_t>(out->splits) * m * n * batch;
+    } else {
+        out->splits = 1;
+        out->kchunk = k;
+        out->tail = 0;
+    }
+    return true;
 }
 
 int launch_x3(int tile, bool br, int ta, int tb, const GemmArgs& g, int batch, hipStream_t stream)

@@ -291,7 +291,9 @@ int attn_bwd(const float* qkv, const float2* cs, const float* P, const float* ct
 //   ws          : split-K.  Shapes with fewer output tiles than CUs and K >= 512
 //                 are split over K into up to 64 slices; partials go to ws and a
 //                 second kernel sums them in slice order (deterministic).
+struct X3Plan;   // lhip_gemm.h
 struct GemmOpts {
+    const X3Plan* plan = nullptr;   // immediate products: planned with their workspace
     int inner = 1;
     long long sA2 = 0, sB2 = 0, sC2 = 0;
     const float* R = nullptr;
@@ -352,7 +354,9 @@ int sgemm_run(int transa, int transb, int m, int n, int k, float alpha,
               float* C, int ldc, long long sC, int batch, const GemmOpts& o, hipStream_t stream);
 // Floats of split-K workspace an immediate product (lhip_sgemm's) asks for,
 // next to `head` floats the caller needs itself.
-size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, size_t head);
+// *plan (may be NULL) receives the split planned for it when *planned is set.
+size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int lda, int ldb, int ldc, size_t head,
+                    X3Plan* plan = nullptr, bool* planned = nullptr);
 
 int sgemm_launch(int transa, int transb, int m, int n, int k, float alpha,
                  const float* A, int lda, const float* B, int ldb, float beta,

@@ -729,7 +729,7 @@ LHIP_API int lhip_gemm_ex(const float* A, const float* B, float* C, const float*
     const size_t post_floats = post ? static_cast<size_t>(M) * N * batch : 0;
     const size_t head = ((pre_floats + 63) & ~static_cast<size_t>(63)) + ((post_floats + 63) & ~static_cast<size_t>(63));
     if (!post && tc) { gm = N; gn = M; gta = !tb; gtb = pre ? 1 : !ta; }
-    const size_t split_need = lhip::immediate_ws(gta, gtb, gm, gn, K, batch, std::max(lda, ldb), std::max(lda, ldb), head);
+    const size_t split_need = lhip::immediate_ws(gta, gtb, gm, gn, K, batch, std::max(lda, ldb), std::max(lda, ldb), gn, head);
     float* work = nullptr;
     if (head + split_need > 0) {
         int rc = lhip::workspace((head + split_need) * sizeof(float), reinterpret_cast<void**>(&work));
