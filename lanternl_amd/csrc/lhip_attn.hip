@@ -32,6 +32,7 @@
 // head h in columns h*hd .. h*hd+hd-1; P[B][H][T][T]; rope table cs[T][hd/2]
 // of (cos, sin) for positions 0..T-1.
 #include <cmath>
+#include <type_traits>
 
 #include "lhip_internal.h"
 #include "lhip_reduce.h"
@@ -678,6 +679,308 @@ __global__ void __launch_bounds__(kAttnThreads) attn_bwd_kernel(const AttnArgs a
     }
 }
 
+// ---- longer windows ---------------------------------------------------------
+// Windows of 65 .. 512 tokens (q and k rotated beforehand): the same products as
+// above with a workgroup of four waves per (window, head, 16-row block) and
+// operands straight from global memory, so nothing but the waves' shares goes
+// through LDS.  The composition they replace (scores, softmax, PV; dP, dv,
+// softmax backward, dq, dk, RoPE) was nine launches that wrote and read the
+// [B, H, T, T] scores four times.  Steps of the whole model, composed and fused:
+// 4000x512x4 on 8x256 tokens (8 heads of 64) 1767 and 1661 us, 2000x128x4 on
+// 4x256 (4 heads of 32) 448 and 354, 500x64x2 on 8x128 184 and 136, 1000x256x2 on
+// 4x512 608 and 525.  Bounded by the loads of the operand blocks (from L2), not
+// by the matrix cores.
+//
+// Forward: wave w takes key blocks w, w + 4, ...; S^T blocks in registers (lane
+// (r, q), element e: query i0 + r, key j0 + 4q + e), row maxima and sums through
+// LDS in wave order, P to global, P . v shares summed in wave order.
+constexpr int kLongMax = 512;
+
+template <int U, int JB>   // hd <= 16 U, T <= 64 JB
+__global__ void __launch_bounds__(kAttnThreads) attn_fwd_long_kernel(const AttnArgs a)
+{
+    __shared__ __align__(16) float part[4][16 * kLd];
+    __shared__ float rmax[4][16], rsum[4][16];
+    const int T = a.T, hd = a.hd, D = a.D;
+    const int nbt = (T + 15) >> 4;
+    const int pid = xcd_pid(blockIdx.x, gridDim.x);
+    const int c = pid % nbt, bh = pid / nbt, b = bh / a.H, h = bh - b * a.H;
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i0 = 16 * c, nj = a.causal ? c + 1 : nbt;
+    const long long ND = static_cast<long long>(a.N) * D;
+    const float* __restrict__ base = a.qkv + static_cast<long long>(b * T) * D + h * hd;
+    const int lim = attn_lim(i0 + r, T, a.causal);
+    float4 qv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int d = 16 * u + 4 * q;
+        qv[u] = *reinterpret_cast<const float4*>(base + static_cast<long long>(min(i0 + r, T - 1)) * D + (d < hd ? d : 0));
+        if (d >= hd) qv[u] = make_float4(0.f, 0.f, 0.f, 0.f);   // k's columns past hd then count for nothing
+    }
+    float sv[JB][4];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < JB; ++t) {
+        const int jb = wave + 4 * t;
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        if (jb < nj) {   // wave-uniform
+            const float* kr = base + ND + static_cast<long long>(min(16 * jb + r, T - 1)) * D;
+            float4 kv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int d = 16 * u + 4 * q;
+                kv[u] = *reinterpret_cast<const float4*>(kr + (d < hd ? d : 0));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const bool in = 16 * u + 4 * q < hd;   // (0 times a non-finite k would not be 0)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[u].x : 0.f, qv[u].x, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[u].y : 0.f, qv[u].y, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[u].z : 0.f, qv[u].z, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? kv[u].w : 0.f, qv[u].w, acc, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            sv[t][e] = (jb < nj && 16 * jb + 4 * q + e < lim) ? acc[e] * a.scale : -INFINITY;
+            mx = fmaxf(mx, sv[t][e]);
+        }
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16));
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    if (q == 0) rmax[wave][r] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(rmax[0][r], rmax[1][r]), fmaxf(rmax[2][r], rmax[3][r]));
+    const float m0 = (mx == -INFINITY || mx != mx) ? 0.f : mx;
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < JB; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int jb = wave + 4 * t;
+            sv[t][e] = (jb < nj && 16 * jb + 4 * q + e < lim) ? expf(sv[t][e] - m0) : 0.f;
+            sum += sv[t][e];
+        }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (q == 0) rsum[wave][r] = sum;
+    __syncthreads();
+    sum = ((rsum[0][r] + rsum[1][r]) + rsum[2][r]) + rsum[3][r];
+    const float is = sum > 0.f ? 1.0f / sum : 1.0f;
+    const int row = i0 + r;
+    float* Pg = a.P + (static_cast<long long>(b) * a.H + h) * T * T + static_cast<long long>(row) * T;
+    floatx4 o[U];
+#pragma unroll
+    for (int db = 0; db < U; ++db) o[db] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < JB; ++t) {
+        const int jb = wave + 4 * t;
+        if (jb < nj) {   // blocks past the causal edge are never read
+            const int j = 16 * jb + 4 * q;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sv[t][e] *= is;
+            if (row < T) {
+                if (a.vec) {
+                    if (j < T) *reinterpret_cast<float4*>(Pg + j) = make_float4(sv[t][0], sv[t][1], sv[t][2], sv[t][3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (j + e < T) Pg[j + e] = sv[t][e];
+                }
+            }
+            float vv[4][U];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int db = 0; db < U; ++db) {
+                    const int d = 16 * db + r;
+                    vv[e][db] = base[2 * ND + static_cast<long long>(min(j + e, T - 1)) * D + (d < hd ? d : 0)];
+                }
+#pragma unroll
+            for (int db = 0; db < U; ++db)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(sv[t][e], vv[e][db], o[db], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int db = 0; db < U; ++db)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[wave][(4 * q + e) * kLd + 16 * db + r] = o[db][e];
+    __syncthreads();
+    const int i = threadIdx.x >> 4, d = 4 * (threadIdx.x & 15);
+    if (i0 + i < T && d < hd) {
+        float4 x = *reinterpret_cast<const float4*>(&part[0][i * kLd + d]);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            const float4 y = *reinterpret_cast<const float4*>(&part[w][i * kLd + d]);
+            x.x += y.x; x.y += y.y; x.z += y.z; x.w += y.w;
+        }
+        *reinterpret_cast<float4*>(a.ctx + static_cast<long long>(b * T + i0 + i) * D + h * hd + d) = x;
+    }
+}
+
+// Backward, the jobs A and B above: wave w takes query blocks w, w + 4, ... past
+// c for dv(c) and dk(c), and key blocks up to c for dq(c).  G = dO v^T comes out
+// of the matrix cores in the layout the next product takes as its A operand
+// (query 4q + e, key r for job A; key 4q + e, query r for job B), and D = rowsum(dO
+// o O) of a block's rows is formed by the wave from the rows it loads anyway.
+template <int U>
+__global__ void __launch_bounds__(kAttnThreads) attn_bwd_long_kernel(const AttnArgs a)
+{
+    __shared__ __align__(16) float part[3][4][16 * kLd];   // per wave: dv, dk, dq shares [row][d]
+    const int T = a.T, hd = a.hd, D = a.D, pairs = hd >> 1;
+    const int nbt = (T + 15) >> 4;
+    const int pid = xcd_pid(blockIdx.x, gridDim.x);
+    const int c = pid % nbt, bh = pid / nbt, b = bh / a.H, h = bh - b * a.H;
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long ND = static_cast<long long>(a.N) * D;
+    const long long head = static_cast<long long>(b * T) * D + h * hd;
+    const float* __restrict__ qp = a.qkv + head;
+    const float* __restrict__ kp = qp + ND;
+    const float* __restrict__ vp = kp + ND;
+    const float* __restrict__ gp = a.dctx + head;
+    const float* __restrict__ op = a.ctx + head;
+    const float* Pg = a.P + (static_cast<long long>(b) * a.H + h) * T * T;
+    // row i0 + r of X, columns 16u + 4q .. +3 (zero past hd and past T)
+    auto frag = [&](const float* __restrict__ X, int i0, float4 (&f)[U]) {
+        const float* x = X + static_cast<long long>(min(i0 + r, T - 1)) * D;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int d = 16 * u + 4 * q;
+            f[u] = *reinterpret_cast<const float4*>(x + (d < hd ? d : 0));
+            if (d >= hd || i0 + r >= T) f[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    // rows i0 + 4q + e of X, column 16 db + r
+    auto cols = [&](const float* __restrict__ X, int i0, float (&x)[4][U]) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int db = 0; db < U; ++db) {
+                const int d = 16 * db + r;
+                x[e][db] = X[static_cast<long long>(min(i0 + 4 * q + e, T - 1)) * D + (d < hd ? d : 0)];
+            }
+    };
+    auto rowdot = [&](const float4 (&x)[U], const float4 (&y)[U]) {
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += x[u].x * y[u].x + x[u].y * y[u].y + x[u].z * y[u].z + x[u].w * y[u].w;
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        return s;
+    };
+    auto product = [&](const float4 (&x)[U], const float4 (&y)[U]) {
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u].x, y[u].x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u].y, y[u].y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u].z, y[u].z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u].w, y[u].w, acc, 0, 0, 0);
+        }
+        return acc;
+    };
+    const int c0 = 16 * c;
+    float4 vc[U], gc[U], oc[U];
+    frag(vp, c0, vc);
+    frag(gp, c0, gc);
+    frag(op, c0, oc);
+    const float Dc = rowdot(gc, oc);   // of query row c0 + r
+    floatx4 dv[U], dk[U], dq[U];
+#pragma unroll
+    for (int db = 0; db < U; ++db) dv[db] = dk[db] = dq[db] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    for (int w = (a.causal ? c : 0) + wave; w < nbt; w += 4) {   // job A: query block w
+        const int i0 = 16 * w;
+        float4 g[U], o[U];
+        float P[4], x[4][U], y[4][U];
+        frag(gp, i0, g);
+        frag(op, i0, o);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = i0 + 4 * q + e;
+            P[e] = Pg[static_cast<long long>(min(i, T - 1)) * T + min(c0 + r, T - 1)];
+            if (i >= T || c0 + r >= T) P[e] = 0.f;
+        }
+        cols(gp, i0, x);
+        cols(qp, i0, y);
+        const float Dr = rowdot(g, o);
+        const floatx4 G = product(g, vc);   // (query 4q + e, key r)
+        float dS[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dS[e] = a.scale * (P[e] * (G[e] - __shfl(Dr, 4 * q + e)));
+#pragma unroll
+        for (int db = 0; db < U; ++db)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                dv[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(P[e], x[e][db], dv[db], 0, 0, 0);
+                dk[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(dS[e], y[e][db], dk[db], 0, 0, 0);
+            }
+    }
+    for (int w = 3 - wave; w < (a.causal ? c + 1 : nbt); w += 4) {   // job B: key block w
+        const int j0 = 16 * w, i = c0 + r;
+        float4 v[U];
+        float P[4], y[4][U];
+        frag(vp, j0, v);
+        const float* Pr = Pg + static_cast<long long>(min(i, T - 1)) * T;
+        if (a.vec) {
+            const float4 t = *reinterpret_cast<const float4*>(Pr + min(j0 + 4 * q, T - 4));
+            P[0] = t.x; P[1] = t.y; P[2] = t.z; P[3] = t.w;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) P[e] = Pr[min(j0 + 4 * q + e, T - 1)];
+        }
+        cols(kp, j0, y);
+        const floatx4 G = product(v, gc);   // (key 4q + e, query r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float p = (i < T && j0 + 4 * q + e < T) ? P[e] : 0.f;
+            P[e] = a.scale * (p * (G[e] - Dc));
+        }
+#pragma unroll
+        for (int db = 0; db < U; ++db)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dq[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(P[e], y[e][db], dq[db], 0, 0, 0);
+    }
+#pragma unroll
+    for (int db = 0; db < U; ++db)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int at = (4 * q + e) * kLd + 16 * db + r;
+            part[0][wave][at] = dv[db][e];
+            part[1][wave][at] = dk[db][e];
+            part[2][wave][at] = dq[db][e];
+        }
+    __syncthreads();
+    // rows c0 .. c0+15: thread (i, g) sums the waves' shares of columns 4g .. 4g+3
+    // in wave order; dq and dk through the inverse RoPE of their two pairs
+    const int i = threadIdx.x >> 4, d = 4 * (threadIdx.x & 15), row = c0 + i;
+    if (row < T && d < hd) {
+        float4 s[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            s[k] = *reinterpret_cast<const float4*>(&part[k][0][i * kLd + d]);
+#pragma unroll
+            for (int w = 1; w < 4; ++w) {
+                const float4 t = *reinterpret_cast<const float4*>(&part[k][w][i * kLd + d]);
+                s[k].x += t.x; s[k].y += t.y; s[k].z += t.z; s[k].w += t.w;
+            }
+        }
+        const float4 cs = *reinterpret_cast<const float4*>(a.cs + row * pairs + (d >> 1));
+        auto back = [&](const float4& x) {
+            return make_float4(x.x * cs.x + x.y * cs.y, -x.x * cs.y + x.y * cs.x, x.z * cs.z + x.w * cs.w,
+                               -x.z * cs.w + x.w * cs.z);
+        };
+        float* o = a.dqkv + head + static_cast<long long>(row) * D + d;
+        *reinterpret_cast<float4*>(o) = back(s[2]);
+        *reinterpret_cast<float4*>(o + ND) = back(s[1]);
+        *reinterpret_cast<float4*>(o + 2 * ND) = s[0];
+    }
+}
+
 }  // namespace
 
 bool attn_fused_ok(int T, int hd) { return T >= 1 && T <= kMax && hd >= 2 && hd <= kMax && hd % 2 == 0; }
@@ -720,6 +1023,58 @@ int attn_bwd(const float* qkv, const float2* cs, const float* P, const float* ct
              aligned16(dqkv)) ? 1 : 0;
     klaunch(attn_bwd_kernel, B * H * ((T + 15) / 16), kAttnThreads, 0, s, a);
     return check_launch("attn_bwd");
+}
+
+bool attn_long_ok(int T, int hd) { return T > kMax && T <= kLongMax && hd >= 4 && hd <= kMax && hd % 4 == 0; }
+
+static AttnArgs long_args(const float* qkv, const float2* cs, float* P, float* ctx, int B, int H, int T, int hd,
+                          float scale, int causal)
+{
+    AttnArgs a{};
+    a.qkv = qkv; a.cs = cs; a.P = P; a.ctx = ctx;
+    a.B = B; a.H = H; a.T = T; a.hd = hd; a.D = H * hd; a.N = B * T;
+    a.scale = scale; a.causal = causal;
+    a.vec = T % 4 == 0 && aligned16(P);   // P rows in float4
+    return a;
+}
+
+// Windows past the limits above: q and k in qkv are already rotated.
+int attn_fwd_long(const float* qkv, float* P, float* ctx, int B, int H, int T, int hd, float scale, int causal,
+                  hipStream_t s)
+{
+    if (!attn_long_ok(T, hd)) return fail(LHIP_E_UNSUPPORTED, "attn_fwd_long: T=%d hd=%d outside its limits", T, hd);
+    if (!qkv || !P || !ctx) return fail(LHIP_E_NULL, "attn_fwd_long: NULL argument");
+    if (!aligned16(qkv) || !aligned16(ctx)) return fail(LHIP_E_ARG, "attn_fwd_long: qkv and ctx must be 16-byte aligned");
+    const AttnArgs a = long_args(qkv, nullptr, P, ctx, B, H, T, hd, scale, causal);
+    const int grid = B * H * ((T + 15) / 16);
+    auto go = [&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        if (T <= 128) klaunch(attn_fwd_long_kernel<U, 2>, grid, kAttnThreads, 0, s, a);
+        else if (T <= 256) klaunch(attn_fwd_long_kernel<U, 4>, grid, kAttnThreads, 0, s, a);
+        else klaunch(attn_fwd_long_kernel<U, 8>, grid, kAttnThreads, 0, s, a);
+    };
+    if (hd <= 16) go(std::integral_constant<int, 1>{});
+    else if (hd <= 32) go(std::integral_constant<int, 2>{});
+    else if (hd <= 48) go(std::integral_constant<int, 3>{});
+    else go(std::integral_constant<int, 4>{});
+    return check_launch("attn_fwd_long");
+}
+
+int attn_bwd_long(const float* qkv, const float2* cs, const float* P, const float* ctx, const float* dctx, float* dqkv,
+                  int B, int H, int T, int hd, float scale, int causal, hipStream_t s)
+{
+    if (!attn_long_ok(T, hd)) return fail(LHIP_E_UNSUPPORTED, "attn_bwd_long: T=%d hd=%d outside its limits", T, hd);
+    if (!qkv || !cs || !P || !ctx || !dctx || !dqkv) return fail(LHIP_E_NULL, "attn_bwd_long: NULL argument");
+    if (!aligned16(qkv) || !aligned16(cs) || !aligned16(ctx) || !aligned16(dctx) || !aligned16(dqkv))
+        return fail(LHIP_E_ARG, "attn_bwd_long: operands must be 16-byte aligned");
+    AttnArgs a = long_args(qkv, cs, const_cast<float*>(P), const_cast<float*>(ctx), B, H, T, hd, scale, causal);
+    a.dctx = dctx; a.dqkv = dqkv;
+    const int grid = B * H * ((T + 15) / 16);
+    if (hd <= 16) klaunch(attn_bwd_long_kernel<1>, grid, kAttnThreads, 0, s, a);
+    else if (hd <= 32) klaunch(attn_bwd_long_kernel<2>, grid, kAttnThreads, 0, s, a);
+    else if (hd <= 48) klaunch(attn_bwd_long_kernel<3>, grid, kAttnThreads, 0, s, a);
+    else klaunch(attn_bwd_long_kernel<4>, grid, kAttnThreads, 0, s, a);
+    return check_launch("attn_bwd_long");
 }
 
 }  // namespace lhip

@@ -284,6 +284,15 @@ int attn_fwd(const float* qkv, const float2* cs, float* P, float* ctx, int B, in
 int attn_bwd(const float* qkv, const float2* cs, const float* P, const float* ctx, const float* dctx, float* dqkv, int B,
              int H, int T, int hd, float scale, int causal, hipStream_t s);
 
+// The same in one launch per direction for windows of 65 .. 512 tokens (head_dim
+// <= 64, a multiple of 4), q and k already rotated in qkv; dq and dk come back
+// through the inverse RoPE.
+bool attn_long_ok(int T, int hd);
+int attn_fwd_long(const float* qkv, float* P, float* ctx, int B, int H, int T, int hd, float scale, int causal,
+                  hipStream_t s);
+int attn_bwd_long(const float* qkv, const float2* cs, const float* P, const float* ctx, const float* dctx, float* dqkv,
+                  int B, int H, int T, int hd, float scale, int causal, hipStream_t s);
+
 // Options of the GEMM launcher.
 //   inner / s?2 : second batch level -- blockIdx.y = outer * inner + i and operand
 //                 X is offset by outer * sX2 + i * sX (e.g. window x head);

@@ -111,6 +111,7 @@ struct LmModel {
     size_t splitk_floats = 0;
     float2* rope_cs = nullptr;    // (cos, sin) of positions 0..T-1, pairs 0..hd/2-1
     bool fused_attn = false;      // per-(window, head) fused attention kernels
+    bool long_attn = false;       // one attention launch per direction past their limits
     bool fused_gemm = false;      // norm / SwiGLU stages fused into their GEMMs
     // graph
     bool use_graph = false;
@@ -277,6 +278,10 @@ int enqueue_step(LmModel& m, hipStream_t s, const Hyper& hp, bool device_hyper)
         } else {
             // RoPE on q and k (2N rows, positions row % T), interleaved pairs
             LM_TRY(rope(qkv, nullptr, 2 * N, H, hd, D, 0, T, base, 1, 0, s));
+        }
+        if (!m.fused_attn && m.long_attn) {
+            LM_TRY(attn_fwd_long(qkv, P, ctx, m.B, H, T, hd, scale, causal, s));
+        } else if (!m.fused_attn) {
             // scores = q_bh . k_bh^T per (window, head), into the (forward-idle) dP
             // scratch; P = softmax(scale * scores)
             LM_TRY(q.hgemm(0, 1, T, T, hd, qkv, D, hd, TD, qkv + ND, D, hd, TD, m.dP, T, TT, HTT));
@@ -410,6 +415,8 @@ int enqueue_step(LmModel& m, hipStream_t s, const Hyper& hp, bool device_hyper)
         if (m.fused_attn) {
             // dP, dv, softmax backward, dq, dk and the inverse RoPE per (window, head)
             LM_TRY(attn_bwd(qkv, m.rope_cs, P, ctx, m.dctx, dqkv, m.B, H, T, hd, scale, causal, s));
+        } else if (m.long_attn) {
+            LM_TRY(attn_bwd_long(qkv, m.rope_cs, P, ctx, m.dctx, dqkv, m.B, H, T, hd, scale, causal, s));
         } else {
             // per (window, head): dP = dO . v^T ; dv = P^T . dO
             LM_TRY(q.hgemm(0, 1, T, T, hd, m.dctx, D, hd, TD, qkv + 2 * ND, D, hd, TD, m.dP, T, TT, HTT));
@@ -733,6 +740,7 @@ LHIP_API int lhip_lm_create(const lhip_lm_config_t* cfg, void** model)
         }
     }
     m->fused_attn = lhip::attn_fused_ok(m->T, m->hd);
+    m->long_attn = lhip::attn_long_ok(m->T, m->hd);
     // The fused 16x16-tile GEMMs save a launch per norm, gate and norm
     // backward; with enough rows the separate kernels and the larger tiles are
     // faster (step, us, fused and separate): dim 128 with 1024 rows 331 and
