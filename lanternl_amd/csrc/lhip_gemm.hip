@@ -1849,10 +1849,14 @@ size_t immediate_ws(int transa, int transb, int m, int n, int k, int batch, int 
 {
     if (planned) *planned = false;
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 0;
+    const bool skinny = skinny_ok(transa, transb, m, n, batch, 1);
+    // the smallest products, whose host time counts: 16x16 tiles, never split
+    if (k <= 1024 && m > 64 && tiny_best(transa, transb, m, n, k, batch, 0, 0) &&
+        static_cast<long long>((m + 31) / 32) * ((n + 31) / 32) * batch < (st().cu_count > 0 ? st().cu_count : 256))
+        return 0;
     const size_t doc = documented_partials(transa, transb, m, n, k, batch);
     size_t need = 0;
     X3Plan p{};
-    const bool skinny = skinny_ok(transa, transb, m, n, batch, 1);
     if (skinny) {
         int kchunk = 0;
         const int s = skinny_plan(m, n, k, static_cast<size_t>(1) << 26, &kchunk);

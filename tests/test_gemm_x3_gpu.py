@@ -20,7 +20,7 @@ SHAPES = [
     (2050, 1999, 33), (1100, 1300, 1025),        # 128x128 tiles, a K remainder of one
     (1024, 1024, 1040), (1025, 1030, 17),        # wave sets with an uneven last round; one stage and one k
     (33, 33, 3000), (20, 20, 5000), (1, 3, 9001),  # one tile, many slices
-    (300, 3000, 300), (65, 4099, 2049),
+    (300, 3000, 300), (65, 4099, 2049), (2000, 2100, 5),
     # the last tiles of a round split over K: a few, nearly half a round, with a
     # K remainder, past several rounds
     (2060, 2050, 768), (1999, 2700, 400), (2060, 2050, 531), (4200, 4200, 1056),
