@@ -274,9 +274,9 @@ sgemm_mfma_ks_kernel(const GemmArgs g)
 }
 
 // ---------------------------------------------------------------------------
-// Skinny products (M <= 64 rows of C, B stored K x N): the work is one
+// Skinny products (M <= 32 rows of C, B stored K x N): the work is one
 // streaming pass over B, HBM-bound.  With one or two rows of C this VALU form
-// streams B (2 to 4 FMAs per float4 of B); three to 64 rows take the MFMA
+// streams B (2 to 4 FMAs per float4 of B); three to 32 rows take the MFMA
 // form below, since at 16 rows the 64 FMAs per float4 outrun the VALU (packed
 // fp32 is not used).  Each wave covers 256 columns with one float4 per lane.  The workgroup walks its K slice in chunks of kSkinnyKC
 // rows: the chunk of A is staged in LDS as [k][m] (zero past M and past the
@@ -410,8 +410,8 @@ sgemm_skinny_kernel(const GemmArgs g)
     }
 }
 
-// Skinny products with 3..64 rows of C on the matrix cores.  The VALU form
-// above would spend up to 64 FMAs per float4 of B, more than the VALU issues at
+// Skinny products with 3..32 rows of C on the matrix cores.  The VALU form
+// above would spend up to 32 FMAs per float4 of B, more than the VALU issues at
 // HBM rate; v_mfma_f32_16x16x4f32 covers 16 rows at once, and MG groups of 16
 // rows (MG = ceil(M / 16)) reuse each float4 of B for 4 * MG MFMAs.  Each wave
 // covers 64 columns: lane (q = l/16, p = l%16) loads the float4
@@ -424,8 +424,8 @@ sgemm_skinny_kernel(const GemmArgs g)
 constexpr int kSkinnyMfmaCols = 64;
 
 // A is staged in LDS per chunk of KC K rows (loading it per step, MG scalar
-// loads a lane per 4-row step each touching 16 rows, outweighed the stream of
-// B at 64 rows and measured 6% slower at 16).  Eight
+// loads a lane per 4-row step each touching 16 rows, measured 6% slower at 16
+// rows).  Eight
 // waves (two per SIMD) take the 4-row steps w, w + 8, ... of a chunk.  A chunk
 // is loaded as float4 along k (thread (m, k4): A[m][kc + 4k4 .. +3]) and written
 // k-major As[k][m] with row stride 80 (16k + m spreads a wave's writes and the
@@ -926,7 +926,7 @@ int launch_tiny(int ta, int tb, GemmArgs g, int batch, hipStream_t stream)
     return launch_reduce(g, batch, stream);
 }
 
-// Skinny path: M <= 64, B not transposed, one product (no batch, no
+// Skinny path: M <= 32, B not transposed, one product (no batch, no
 // batch-reduce), at least one full wave of columns.
 bool skinny_ok(int ta, int tb, int m, int n, int batch, int kblocks)
 {
@@ -934,7 +934,7 @@ bool skinny_ok(int ta, int tb, int m, int n, int batch, int kblocks)
     return !tb && m >= 1 && m <= kSkinnyMax && n >= kSkinnyCols && batch == 1 && kblocks == 1;
 }
 
-// Rows of C up to which the VALU form is used; 3..64 rows take the MFMA form.
+// Rows of C up to which the VALU form is used; 3..32 rows take the MFMA form.
 constexpr int kSkinnyValuMax = 2;
 
 }  // namespace
@@ -947,7 +947,7 @@ int skinny_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
     const int cus = st().cu_count > 0 ? st().cu_count : 256;
     const long long cb = ceil_div(n, m <= kSkinnyValuMax ? kSkinnyCols : kSkinnyMfmaCols);
     // about two workgroups per CU for the VALU form and the one-group (M <= 16)
-    // MFMA form; one for the eight-wave MFMA form on 2-4 groups (M = 4, 8, 16
+    // MFMA form; one for the eight-wave MFMA form on two groups (M = 4, 8, 16
     // at K = N = 4096: 24.1, 24.5, 21.1 us on one per CU, 19.6, 19.6, 19.3 on
     // two; M = 32: 29.2 on one, 30.7 on two)
     const long long per_cu = m <= 16 ? 2 : 1;
@@ -1665,8 +1665,8 @@ int tiny_unreduced_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
 // with K up to 256, or 512 for the first quarter past one (512x640x256 NN 6.0 us
 // against 8.5, 512x512x512 8.5 against 12.1, 521x665x186 TN 6.8 against 9.3, but
 // unaligned NT 8.9 against 7.2; 800x800x130, 2.4 tiles per CU, 8.9 against 7.5).
-// With fewer tiles than CUs K up to 1024; up to 2048 when both operands take float4 loads (256x256x1536 NT 11.1
-// us against 12.1 on the three-term kernel, 512x128x2000 10.2 against 11.6;
+// With fewer tiles than CUs K up to 1024; up to 2048 when both operands take
+// float4 loads (256x256x1536 NT 11.1 us against 12.1 on the three-term kernel, 512x128x2000 10.2 against 11.6;
 // unaligned 238x474x1199 28.4 against 12.4); up to 4096 where B is read along
 // its rows and the product is one column tile wide, or A is K-major
 // (4096x16x4096 NN 21.2 against 25.0, TN 23.2 against 31.0; 128x128x4096 TN

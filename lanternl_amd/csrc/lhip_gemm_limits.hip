@@ -44,7 +44,6 @@ int ks_split_plan(int m, int n, int k, size_t ws_floats, int* kchunk_out)
 // the 64x64 tiles (+ split-K) save in latency.
 bool use_small_kernel(int m, int n, int k) { return k <= 2048 || m <= 64 || n <= 64; }
 
-
 // 256x256 tiles split over K (one batch): when the tiles alone would fill
 // between a quarter and all of the CUs (e.g. 2048^3: 64 tiles), each tile's K
 // is cut into slices of at least 512 so that tiles x slices covers the CUs;

@@ -76,12 +76,12 @@ __device__ __forceinline__ void split_pair(float x, float y, unsigned& h, unsign
 //
 // A unit is KW consecutive k of one row.  Row-contiguous operands load a unit
 // with one 16-byte load (four lanes cover a row's 64 bytes); K-major ones load
-// a dword per k, 64 consecutive rows per wave, so no alignment or width is
-// asked of N or ld.  In LDS each term is a plane of two halves (k 0-7, 8-15)
+// a dword per k (consecutive lanes on consecutive rows; with four k per unit,
+// lane pairs share a row), so no alignment or width is asked of N or ld.  In LDS each term is a plane of two halves (k 0-7, 8-15)
 // of ROWS x 8 bf16: an MFMA fragment is one ds_read_b128 of 32 consecutive
-// 16-byte rows per half wave.  The halves are 128 bytes apart modulo the 256
-// bytes of banks, so the row-contiguous units' ds_write_b64 (8 rows x 2 halves
-// per half wave) cover every bank once; the K-major units write whole
+// 16-byte rows per half wave.  The halves are 64 bytes apart modulo
+// 128, so 16 lanes of ds_write_b64 (4 rows x 2 halves of row-contiguous units)
+// write 128 different bytes of banks; K-major units of eight k write whole
 // 16-byte rows.
 template <int ROWS, int NT, bool KMAJOR>
 struct X3Stage {
@@ -625,7 +625,7 @@ struct X3Tile {
     double fixed, alone, shared;
 };
 constexpr X3Tile kX3Tiles[] = {
-    {256, 10.0, 1.68, 1.90},   // 8 waves of 128x64: 41% of the bf16 peak at 4096^3, where power limits it
+    {256, 10.0, 1.68, 1.90},   // 8 waves of 128x64: 53-57% of the bf16 peak at 4096^3 (220-237 TFLOP/s x 6), where power limits it
     {128, 6.0, 0.53, 0.62},    // 8 waves of 64x32, two workgroups per CU
     {128, 8.0, 0.455, 0.0},    // 2 wave sets of 64x64 waves, one workgroup per CU
     {64, 5.5, 0.25, 0.225},    // 2 wave sets of 32x32 waves
